@@ -7,9 +7,9 @@
 // configuration (F2Tune) that the plan carries: the work-item schedule over the dies,
 // the FP64 kernel's wavefront tile (64 x 64 or 32 x 64 outputs), whether it prefetches
 // the next K-step, the FP64 and pair-count grids.  The split kernel's tile is fixed by
-// its LDS ring (one 128 x 128 workgroup per CU); its schedule, the count grid and the
-// placement of its global-to-LDS loads (a burst after each phase barrier, or one at a
-// time between the phase's MFMAs) are tuned.  f2_autotune times every candidate on the caller's device inputs (every
+// its LDS ring (one 128 x 128 workgroup per CU); its schedule, the count grid and the order
+// of its LDS reads (the compiler's, or each left fragment one product group ahead) are
+// tuned.  f2_autotune times every candidate on the caller's device inputs (every
 // candidate writes bit-identical tensors: the same sums per entry, in the same order),
 // keeps the fastest per key — device name, precision, P, and the block-size histogram
 // (blocks per power-of-two padded length) — and saves the table to a text file

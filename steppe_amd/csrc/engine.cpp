@@ -373,10 +373,12 @@ void HipBackend::run_f2(const F2Plan& plan, int precision, const F2Source& src, 
     };
     // The pair-count kernel runs one 128x128 item per 4-wavefront workgroup.
     const int n_wg_count = grid(tn.count_wg_per_cu, 4 * static_cast<std::int64_t>(plan.items128.size()));
-    w.planeV8.ensure(std::max<std::size_t>(plane, 16));
-    // queue cursors of the two kernels, then one item word per split workgroup
-    w.counters.ensure(2 * kXcds + kMaxSplitWorkgroups);
+    // queue cursors of the two kernels
+    w.counters.ensure(2 * kXcds);
+    const std::int64_t KS32 = plan.K_total / 32;
+    const std::size_t plane32 = static_cast<std::size_t>(plan.G32) * 32 * static_cast<std::size_t>(plan.K_total);
     if (precision == STP_PREC_FP64) {
+        w.planeV8.ensure(std::max<std::size_t>(plane32, 16));
         w.planeA.ensure(std::max<std::size_t>(plane, 1));
         w.planeV.ensure(std::max<std::size_t>(plane, 1));
         w.planeQ.ensure(std::max<std::size_t>(plane, 1));
@@ -390,8 +392,8 @@ void HipBackend::run_f2(const F2Plan& plan, int precision, const F2Source& src, 
                                  w.planeA.get(), w.planeV.get(), w.planeQ.get(), w.planeV8.get(), stream_);
         mark_end(kPrep);
         mark_begin(kCount);
-        launch_count(w.planeV8.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get(), plan.P, plan.G,
-                     plan.K_total / 64, d_vpair, n_wg_count, stream_);
+        launch_count_v8(w.planeV8.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get(), plan.P, plan.G32, KS32,
+                        d_vpair, n_wg_count, stream_);
         mark_end(kCount);
         const FixupList fl = fixup_list(plan, kFixupTauFp64, w);
         const int units = n_items * (tn.fp64_rows == 32 ? 2 : 1);
@@ -404,30 +406,28 @@ void HipBackend::run_f2(const F2Plan& plan, int precision, const F2Source& src, 
         run_fixup(plan, src, fl, d_f2, d_vpair, w);
         return;
     }
-    // Split-BF16: 13 digit planes of 2 bytes per (row, SNP), rows padded to 32.
-    const std::int64_t KS16 = plan.K_total / 16;
-    const std::size_t split_bytes = static_cast<std::size_t>(plan.G32) * 32 * plan.K_total * 2 * kSplitPlanes;
-    w.planeSplit.ensure(std::max<std::size_t>(split_bytes, 16));
+    // Split form: 12 one-byte digit planes, rows padded to 32.
+    // (at least one K-step of one row group: what an empty partition's prologue reads)
+    w.planeSplit.ensure(kSplitPlanes * std::max<std::size_t>(plane32, 1024));
     mark_begin(kPrep);
     if (src.a2)
-        launch_prep_split_counts(src.a2, src.n, src.ld, plan.P, plan.G32, plan.G, bt, w.plan.chunk_block.get(),
-                                 n_chunks, KS16, w.planeSplit.get(), w.planeV8.get(), stream_);
+        launch_prep_split_counts(src.a2, src.n, src.ld, plan.P, plan.G32, bt, w.plan.chunk_block.get(), n_chunks, KS32,
+                                 w.planeSplit.get(), stream_);
     else
-        launch_prep_split_qvn(src.q, src.v, src.nq, plan.P, plan.G32, plan.G, bt, w.plan.chunk_block.get(), n_chunks,
-                              KS16, w.planeSplit.get(), w.planeV8.get(), stream_);
+        launch_prep_split_qvn(src.q, src.v, src.nq, plan.P, plan.G32, bt, w.plan.chunk_block.get(), n_chunks, KS32,
+                              w.planeSplit.get(), stream_);
     mark_end(kPrep);
     mark_begin(kCount);
-    launch_count(w.planeV8.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get(), plan.P, plan.G,
-                 plan.K_total / 64, d_vpair, n_wg_count, stream_);
+    launch_count_split(w.planeSplit.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get(), plan.P, plan.G32,
+                       KS32, d_vpair, n_wg_count, stream_);
     mark_end(kCount);
     const int n_items128 = static_cast<int>(plan.items128.size());
     const FixupList fl = fixup_list(plan, kFixupTauSplit, w);
     mark_begin(kF2);
     launch_f2_split(w.planeSplit.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get() + kXcds, plan.P,
-                    plan.G32, KS16, d_vpair, d_f2, fl,
-                    std::min(kMaxSplitWorkgroups,
-                             static_cast<int>(round_up(std::max(1, std::min(n_cu_, n_items128)), kXcds))),
-                    tn.split_ring, reinterpret_cast<int*>(w.counters.get() + 2 * kXcds), stream_);
+                    plan.G32, KS32, d_vpair, d_f2, fl,
+                    static_cast<int>(round_up(std::max(1, std::min(n_cu_, n_items128)), kXcds)), tn.split_ring,
+                    stream_);
     mark_end(kF2);
     run_fixup(plan, src, fl, d_f2, d_vpair, w);
 }

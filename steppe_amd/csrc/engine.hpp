@@ -49,17 +49,21 @@ void launch_f2_fp64(const double* pA, const double* pV, const double* pQ, BlockT
                     const double* vpair, const FixupList& fl, int n_workgroups, int wave_rows, bool prefetch,
                     hipStream_t st);
 void launch_prep_split_counts(const std::uint16_t* a2, const std::uint16_t* n, std::int64_t ld, int P, int G32,
-                              int G16, BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks,
-                              std::int64_t KS16, std::uint8_t* planes, void* pV8, hipStream_t st);
-void launch_prep_split_qvn(const double* q, const double* v, const double* n, int P, int G32, int G16,
-                           BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks, std::int64_t KS16,
-                           std::uint8_t* planes, void* pV8, hipStream_t st);
-void launch_count(const void* pV8, BlockTable bt, const F2Item* items, const ItemQueues& queues,
-                  unsigned* counters, int P, int G16, std::int64_t KS64, double* vpair, int n_workgroups,
-                  hipStream_t st);
+                              BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks,
+                              std::int64_t KS32, std::uint8_t* planes, hipStream_t st);
+void launch_prep_split_qvn(const double* q, const double* v, const double* n, int P, int G32, BlockTable bt,
+                           const std::int32_t* chunk_block, std::int64_t n_chunks, std::int64_t KS32,
+                           std::uint8_t* planes, hipStream_t st);
+// Pair counts from the split form's digit planes, or from the FP64 form's V plane.
+void launch_count_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
+                        unsigned* counters, int P, int G32, std::int64_t KS32, double* vpair, int n_workgroups,
+                        hipStream_t st);
+void launch_count_v8(const std::uint8_t* v8, BlockTable bt, const F2Item* items, const ItemQueues& queues,
+                     unsigned* counters, int P, int G32, std::int64_t KS32, double* vpair, int n_workgroups,
+                     hipStream_t st);
 void launch_f2_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
-                     unsigned* counters, int P, int G32, std::int64_t KS16, const double* vpair, double* f2,
-                     const FixupList& fl, int n_workgroups, int ring, int* item_slot, hipStream_t st);
+                     unsigned* counters, int P, int G32, std::int64_t KS32, const double* vpair, double* f2,
+                     const FixupList& fl, int n_workgroups, int ring, hipStream_t st);
 void launch_f2_fixup_counts(const std::uint16_t* a2, const std::uint16_t* n, std::int64_t ld, BlockTable bt,
                             const FixupList& fl, int P, int n_block, const double* vpair, double* f2,
                             int n_workgroups, hipStream_t st);
@@ -87,10 +91,6 @@ struct NoallocScratch {
 NoallocScratch resolve_noalloc_scratch();
 void launch_ploidy_from_i32(const std::int32_t* in, std::int64_t n, std::int8_t* out, hipStream_t st);
 
-// Upper bound on the split contraction's grid (one workgroup per CU; the per-workgroup
-// item words of its second ring layout live after the queue cursors).
-constexpr int kMaxSplitWorkgroups = 4096;
-
 // ---- launch configuration chosen by the autotuner (autotune.cpp) -----------------------
 struct F2Tune {
     int sched = 0;            // work items: 0 per-die queues (blocks longest-first onto the
@@ -99,8 +99,8 @@ struct F2Tune {
     int fp64_prefetch = 1;    // FP64: load the next K-step while this one's MFMAs run
     int fp64_wg_per_cu = 2;   // FP64 contraction workgroups (4 wavefronts) per CU
     int count_wg_per_cu = 2;  // pair-count kernel workgroups per CU
-    int split_ring = 0;       // split contraction LDS ring: 0 (A, V double-buffered, 152 KB) or
-                              // 1 (A, V, B double-buffered, 160 KB)
+    int split_ring = 0;       // split contraction's reads of its LDS ring: 0 in the compiler's
+                              // order, 1 each left fragment one product group ahead
     std::string str() const;
     static bool parse(const std::string& s, F2Tune& out);
 };
@@ -136,8 +136,8 @@ struct F2Work {
     };
     PlanDev plan;
     DevBuf<double> planeA, planeV, planeQ;      // FP64 operand planes
-    DevBuf<std::uint8_t> planeV8;               // int8 V plane (pair counts)
-    DevBuf<std::uint8_t> planeSplit;            // split-BF16 digit planes
+    DevBuf<std::uint8_t> planeV8;               // FP64 form: int8 V plane (pair counts)
+    DevBuf<std::uint8_t> planeSplit;            // split-form digit planes
     DevBuf<unsigned> counters;                  // work-queue cursors: pair counts, contraction
     DevBuf<unsigned> fix_count;                 // cancellation-prone entries flagged
     DevBuf<std::int32_t> fix_entries;

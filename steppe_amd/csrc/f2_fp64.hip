@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void prep_fp64_kernel(
     }
 
     const std::int64_t t0 = kg0 / 4;  // first 4-column K-step of the chunk
-    const std::int64_t u = c;         // 64-column step index of the int8 plane
+    const std::int64_t u = c;         // 64-column pair of K-steps of the int8 plane
     // Element i of this thread in a group's stage: lanes run along the source's
     // contiguous axis, so every row (or column) segment is read once, coalesced.
     auto elem = [&](int i, int& rr, int& kk) {
@@ -204,13 +204,16 @@ __global__ __launch_bounds__(256) void prep_fp64_kernel(
             unsigned w[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int j = 0; j < 16; ++j)
-                if (sV[rr * kLd + kb + j] != 0.0) w[j >> 2] |= 1u << (8 * (j & 3));
+                if (sV[rr * kLd + kb + j] != 0.0) w[j >> 2] |= 0x40u << (8 * (j & 3));
             i4 v;
             v[0] = static_cast<int>(w[0]);
             v[1] = static_cast<int>(w[1]);
             v[2] = static_cast<int>(w[2]);
             v[3] = static_cast<int>(w[3]);
-            pV8[(static_cast<std::int64_t>(g) * (KS / 16) + u) * 64 + tid] = v;
+            // 16 SNPs kb of row rr: K-step 2u + kb/32, half (kb/16)%2 of a 32-row fragment
+            const int piece = tid >> 4;
+            pV8[(static_cast<std::int64_t>(g >> 1) * (KS / 8) + 2 * u + (piece >> 1)) * 64 + 32 * (piece & 1) +
+                16 * (g & 1) + rr] = v;
         }
         lds_barrier();  // every reader of this group's stage is done
 #pragma unroll

@@ -12,13 +12,13 @@
 //
 //   FP64 planes (v_mfma_f64_16x16x4f64, 4-SNP K-steps, KS = K_total/4 steps):
 //     plane[(g*KS + t)*64 + lane],  lane -> row 16g + lane%16, SNP 4t + lane/16
-//   int8 V plane (v_mfma_i32_16x16x64_i8, 64-SNP K-steps, KS64 = K_total/64):
-//     v8[(g*KS64 + u)*64 + lane] is 16 bytes: row 16g + lane%16,
-//     SNPs 64u + 16*(lane/16) + 0..15
+//   int8 planes (v_mfma_i32_32x32x32_i8, 32-SNP K-steps, KS32 = K_total/32, 32-row groups
+//   g32): the split form's digits and the FP64 form's V plane (bit 6 of a byte = observed):
+//     16 bytes per lane: row 32 g32 + lane%32, SNPs 32 t + 16*(lane/32) + 0..15
 //
 // The same fragment serves as the A operand (rows of the left population tile)
 // and the B operand (rows of the right tile), because both MFMA operand layouts
-// put the output index on lane%16 and the K index on lane/16.
+// put the output index on the low lane bits and the K index on the high ones.
 #pragma once
 
 #include <cstdint>
@@ -28,8 +28,12 @@ namespace stp {
 constexpr int kRowGroup = 16;
 constexpr int kKPad = 64;   // padded block granularity (SNPs)
 constexpr int kTileRows = 64;  // rows per wavefront output tile (4 row groups)
-// Split form: 11 digit planes of 2 bytes per (population, SNP) (f2_split.hip).
-constexpr int kSplitPlanes = 11;
+// Split form: 12 one-byte digit planes per (population, SNP) (f2_split.hip).
+constexpr int kSplitPlanes = 12;
+// Bytes per (population, SNP) that the automatic output tier counts for the split form's
+// working set: more than the planes take, kept so that a panel's tier does not depend on
+// how the digits are laid out.
+constexpr int kSplitTierBytes = 22;
 
 struct BlockTable {
     std::int64_t* s0;    // first SNP of block b

@@ -1,52 +1,50 @@
-// steppe_amd/csrc/f2_split.hip — per-block f2 from fixed-point digit slices on BF16 and
-// FP16 MFMA.
+// steppe_amd/csrc/f2_split.hip — per-block f2 from fixed-point 8-bit digits on int8 MFMA.
 //
 // The reference's default precision is cuBLAS's closed FP64 emulation on integer
 // units (src/device/cuda/f2_block_kernel.cu:121-144).  This is an independent
 // construction from the published Ozaki-scheme idea (Ozaki, Ogita, Oishi & Rump,
 // Numer. Algorithms 59:95-118, 2012; Ootomo, Ozaki & Yokota, IJHPCA 2024): split
 // every operand into fixed-point digits whose pairwise products and partial sums
-// are exact in the MFMA's FP32 accumulator, and recombine the exact partial sums
+// are exact in the MFMA's int32 accumulator, and recombine the exact partial sums
 // in FP64.  It computes the same estimator as the FP64 path (f2_fp64.hip):
 //
 //   num_ij = sum_s v_i v_j [(q_i - q_j)^2 - h_i - h_j],  f2 = num / vpair
 //
 // Operands.  The estimator only sees differences q_i - q_j, so any per-SNP shift of q
 // leaves it unchanged; with q' = q - 1/2 (|q'| <= 1/2) and w = -(q'^2 - h)/2
-// (|w| <= 1/8):
-//   q' is written as six balanced 8-bit digits (|digit| <= 128, exact in BF16),
-//       q~ = 2^-7 sum_k d_k 2^-8k,  k = 0..5;
-//   w (computed from q~, not q') as four FP16 digits of up to 11 significant bits,
-//       w~ = A 2^-14 + B 2^-30 + C 2^-38 + D 2^-46,
-//       A = rint(w 2^14) (|A| <= 2048), B = 32 b, C = 4 c (|b|, |c| <= 1024), |D| <= 512,
-//   so |w - w~| <= 2^-47, and each digit is an integer in the units of the level it
-//   enters.  The device evaluates the estimator for the perturbed frequencies q~
-//   (|q~ - q'| <= 2^-48).  Then, with level units U_t = 2^(-14-8t),
-//     -num_ij / 2 = sum_s [ q~_i q~_j + w~_i v_j + v_i w~_j ] = sum_t U_t * L_t,
-//     L_t = sum_s [ sum_{k+l=t} d_k(i) d_l(j) + W_t(i) v(j) + v(i) W_t(j) ],
-//   W_0 = A, W_1 = 0, W_2 = B, W_3 = C, W_4 = D.
-// The digit products d_k d_l run on BF16 MFMA and the W_t v products on FP16 MFMA
-// (v in {0, 1}); both accumulate into the same FP32 level accumulators.  Levels
-// t = 0..4 each have one.  Per SNP, |L_2| grows by at most 3 * 2^15 and the others by
-// less, so 128 SNPs keep every L_t below 2^24 and the MFMA sums are exact.
-// Level 5 (d_k d_{5-k} for k = 0..5) is folded into L_4 through operands scaled by
-// 2^-8 (exact in BF16): those sums are rounded at 2^-47 per MFMA, far below the
-// result's precision.  Products with k + l >= 6 are dropped (<= 2^-45 per SNP).
-// Every 128 SNPs each level carries its multiple of 2^8 into the level above (exact
-// FP32 operations) and L_0 carries multiples of 2^12 into an FP32 high word, so a
-// block of any length accumulates in six FP32 words per output and FP64 appears only
-// in the per-block epilogue.
+// (|w| <= 1/8), both as 48-bit integers in six balanced 8-bit digits:
+//   q~ = 2^-7 sum_k d_k 2^-8k,           |q~ - q'| <= 2^-48;
+//   w~ = -128 sum_k W_k 2^(-14-8k)       (computed from q~), |w~ - w| <= 2^-48.
+// With level units U_t = 2^(-14-8t) and V = -128 v,
+//   -num_ij / 2 = sum_s [ q~_i q~_j + w~_i v_j + v_i w~_j ] = sum_t U_t * L_t,
+//   L_t = sum_s [ sum_{k+l=t} d_k(i) d_l(j) + W_t(i) V(j) + V(i) W_t(j) ],  t = 0..5.
+// Products with k + l >= 6 are dropped (<= 2^-45 per SNP).
 //
-// MFMA work per (pair, SNP): 29 products (21 BF16 digit-by-digit, 8 FP16
-// digit-by-V), plus the pair count V V^T, computed exactly by a separate int8 MFMA
-// kernel.  Operand bytes per (population, SNP): 22 (six q digits, four w digits, V).
+// V has no plane of its own: |W_0| <= 16, so W_0 + 96 is stored for an observed entry (a
+// byte in [79, 113]: bit 6 is set) and 0 for a missing one, and V = -128 v is the byte
+// (W_0' << 1) & 0x80.  The offset adds 96 (v_i V_j + V_i v_j) = -24576 v_i v_j per SNP
+// to L_0, which the epilogue takes back from the pair count, in integers.
+//
+// Per SNP, |L_5| grows by at most 2*64*128 + 4*2^14 + 2*2^14 = 114,688 and the others by
+// less, so 16,384 SNPs keep every level below 2^31: a block accumulates in six int32
+// words per output with no carries, and FP64 appears only in the epilogue.  Longer blocks
+// are summed in segments of 16,384 SNPs, whose FP64 partial sums meet in the f2 tensor.
+//
+// MFMA work per (pair, SNP): 33 int8 products (21 digit by digit, 12 digit by V) at twice
+// the BF16 rate, plus the pair count V V^T in a kernel of its own.  Operand bytes per
+// (population, SNP): 12.  (The same scheme on BF16 / FP16 digits with FP32 accumulators
+// took 29 products at the BF16 rate, 22 bytes, and carries every 128 SNPs.)
 //
 // Kernel shape: persistent workgroups of 8 wavefronts (2 per SIMD) own a 128x128
 // output tile of one jackknife block; each wavefront owns 64x32 (two 32x32 MFMA
-// tiles, six FP32 accumulators per output).  Each 16-SNP K-step is staged through
-// LDS in two phases by direct global->LDS loads: the q digits (two slots, alternating
-// between K-steps), then the w digits and V (A, V and, in the second ring layout, B in
-// two alternating slots; the rest in one).
+// tiles, six int32 accumulators per output).  Each 32-SNP K-step is two phases (the q
+// digits, then the w digits) whose 48 KB of planes arrive in a ring of three LDS slots
+// by direct global->LDS loads, issued two phases ahead.
+//
+// Bound and measured (1000 populations x 597,573 SNPs, one pass): the contraction issues
+// 33 x 2 ops per pair-SNP of its 128-row tiles, 2.3e13 in 9.2 ms = 2.5 POP/s, the rate an
+// 8192^3 int8 library product reaches on this card (2.49); on the BF16 / FP16 digits it
+// took 18.3 ms.  Prep writes 12 instead of 23 bytes per entry: 2.0 instead of 4.5 ms.
 
 #include <utility>
 
@@ -59,26 +57,19 @@ void launch_zero_u32(unsigned* p, int n, hipStream_t st);
 
 namespace {
 
-typedef float f16v __attribute__((ext_vector_type(16)));
 typedef int i4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef int i16v __attribute__((ext_vector_type(16)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
-constexpr int kPlanes = kSplitPlanes;  // d0..d5 (0-5), w digit A (6), V (7), w digits B, C, D (8-10)
-constexpr int kPlaneA = 6, kVPlane = 7;
-constexpr int kChunk = 1024;           // bytes per (32-row group, 16-SNP step, plane)
+constexpr int kPlanes = kSplitPlanes;  // d0..d5 (0-5), W0'..W5 (6-11)
+constexpr int kSetPlanes = 6;          // planes of one phase: the q digits or the w digits
+constexpr int kChunk = 1024;           // bytes per (32-row group, 32-SNP step, plane)
 constexpr int kGroups = 8;             // 32-row groups per workgroup tile: 4 left + 4 right
-constexpr int kDPlanes = 6;                                 // q digits d0..d5 per slot
-constexpr int kDSlotBytes = kGroups * kDPlanes * kChunk;    // 48 KB
-// The w-digit and V planes in two slot kinds, X (double-buffered) and Y (single), for two
-// ring layouts: RING 0 holds A, V in X and B, C, D in Y (152 KB of LDS in all, the item
-// index broadcast through LDS); RING 1 holds A, V, B in X and C, D in Y (160 KB, all of
-// the LDS, so the item index goes through a per-workgroup word in device memory).
-template <int RING>
-constexpr int x_planes() { return RING ? 3 : 2; }
-template <int RING>
-constexpr int y_planes() { return RING ? 2 : 3; }
+constexpr int kSlotBytes = kGroups * kSetPlanes * kChunk;   // 48 KB
 constexpr int kWaves = 8;
+constexpr int kW0Offset = 96;                               // W_0' - W_0 of an observed entry
+constexpr int kL0PerPair = 2 * 128 * kW0Offset;             // what it takes from L_0 per pair and SNP
+constexpr int kSegSteps = 512;                              // K-steps whose level sums fit int32
 
 // f(std::integral_constant<int, I>) for I = 0 .. N-1, as straight-line code.
 template <int N, class F>
@@ -89,23 +80,52 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // ---------------------------------------------------------------------------------
-// prep: frequencies -> 11 digit planes (32x32x16 MFMA fragment order: six BF16 q
-// digits, then FP16 A, V, B, C, D) + the int8 V plane (16x16x64 fragment order, for
-// the count kernel), in one pass.
-//   plane chunk (g32, t16, p) holds rows 32 g32 + lane%32, SNPs 16 t16 + 8 (lane/32) + j
-//   at byte offset ((g32 * KS16 + t16) * 11 + p) * 1024 + lane * 16 + 2 j.
-//   Plane 5 (d5) is stored scaled by 2^-8 (it only enters level 5).
-// A workgroup converts one (32-row group, 64-SNP chunk) unit at a time: it stages the
-// unit's frequencies and heterozygosity terms in LDS with coalesced row reads, then
-// every thread expands one 8-SNP fragment into its digits.
+// prep: frequencies -> 12 digit planes in 32x32x32 MFMA fragment order, in one pass:
+//   plane chunk (g32, t32, p) holds rows 32 g32 + lane%32, SNPs 32 t32 + 16 (lane/32) + j
+//   at byte offset ((g32 * KS32 + t32) * 12 + p) * 1024 + lane * 16 + j.
+// A workgroup converts one (32-row group, 64-SNP chunk) unit at a time: it stages each
+// entry's two 48-bit integers in LDS (12 bytes, from coalesced row reads), then every
+// thread transposes the bytes of one 16-SNP fragment of the q or the w digits into six
+// 16-byte stores.
 // ---------------------------------------------------------------------------------
-constexpr int kStageLd = 65;  // LDS row stride (doubles) of the staged unit
+constexpr int kStageLd = 65;  // LDS row stride (dwords) of the staged unit
+
+// The staged unit: per entry bytes 0-3 of the q integer, its bytes 4-5 with the w
+// integer's bytes 4-5 above them, bytes 0-3 of the w integer.
+struct Stage {
+    unsigned q[32 * kStageLd];
+    unsigned t[32 * kStageLd];
+    unsigned w[32 * kStageLd];
+};
+
+// An integer |x| < 2^47 given as a double (rounded to nearest even): its balanced digits
+// in bytes 0 (least significant) to 4, each in [-128, 127], and the rest in byte 5.
+// Adding 1.5 * 2^52 leaves the integer in the low bits; adding 128 to every lower digit
+// place makes plain bytes of the balanced digits, and flipping each top bit undoes it.
+__device__ inline unsigned long long balanced48(double x) {
+    const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(x + 0x1.8p52));
+    return (bits + 0x8080808080ull) ^ 0x8080808080ull;
+}
+
+// Stage one entry; h < 0 or NaN (a frequency outside [0, 1]) counts as missing.
+__device__ inline void stage_entry(Stage& st, int at, bool ok, double q, double nm1) {
+    unsigned long long Q = 0, W = 0;
+    const double h = q * (1.0 - q) / (nm1 > 1.0 ? nm1 : 1.0);
+    if (ok && h >= 0.0) {
+        const double x = (q - 0.5) * 0x1p47;
+        const double qt = ((x + 0x1.8p52) - 0x1.8p52) * 0x1p-47;
+        Q = balanced48(x);
+        W = balanced48((qt * qt - h) * 0x1p46) + (static_cast<unsigned long long>(kW0Offset) << 40);
+    }
+    st.q[at] = static_cast<unsigned>(Q);
+    st.t[at] = (static_cast<unsigned>(Q >> 32) & 0xFFFFu) | (static_cast<unsigned>(W >> 32) << 16);
+    st.w[at] = static_cast<unsigned>(W);
+}
 
 // Staging reads of the two frequency sources.  Each thread stages 8 elements of the
 // 32 x 64 unit: fetch() issues the global loads into registers (so a workgroup can
-// fetch its next unit while it converts the current one), put() turns them into
-// (q - 1/2, h) in sq/sh, with h = -1 marking an invalid entry.
-// h = q(1-q)/max(n-1, 1) as in the reference's het_correction
+// fetch its next unit while it converts the current one), put() turns them into staged
+// entries with h = q(1-q)/max(n-1, 1) as in the reference's het_correction
 // (src/core/internal/f2_estimator.hpp:22-29).
 struct CountsSrc {
     const std::uint16_t* a2;
@@ -135,21 +155,15 @@ struct CountsSrc {
         }
         return raw;
     }
-    __device__ void put(const Raw& raw, int tid, double* sq, double* sh) const {
+    __device__ void put(const Raw& raw, int tid, Stage& st) const {
         const int kk = tid & 63;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int row = (tid >> 6) + 4 * i;
-            double qp = 0.0, h = -1.0;
-            if (raw.ok[i] && raw.c[i]) {
-                const double nd = static_cast<double>(raw.c[i]);
-                const double q = static_cast<double>(raw.a[i]) / (2.0 * nd);
-                const double nm1 = nd - 1.0;
-                h = q * (1.0 - q) / (nm1 > 1.0 ? nm1 : 1.0);
-                qp = q - 0.5;
-            }
-            sq[row * kStageLd + kk] = qp;
-            sh[row * kStageLd + kk] = h;
+            const double nd = static_cast<double>(raw.c[i]);
+            const bool ok = raw.ok[i] && raw.c[i];
+            const double q = static_cast<double>(raw.a[i]) / (ok ? 2.0 * nd : 1.0);
+            stage_entry(st, row * kStageLd + kk, ok, q, nd - 1.0);
         }
     }
 };
@@ -180,20 +194,12 @@ struct QvnSrc {
         }
         return raw;
     }
-    __device__ void put(const Raw& raw, int tid, double* sq, double* sh) const {
+    __device__ void put(const Raw& raw, int tid, Stage& st) const {
         const int row = tid & 31;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int kk = (tid >> 5) + 8 * i;
-            double qp = 0.0, h = -1.0;
-            if (raw.ok[i] && raw.v[i] != 0.0) {
-                const double qq = raw.q[i], nm1 = raw.n[i] - 1.0;
-                h = qq * (1.0 - qq) / (nm1 > 1.0 ? nm1 : 1.0);
-                qp = qq - 0.5;
-            }
-            sq[row * kStageLd + kk] = qp;
-            sh[row * kStageLd + kk] = h;
-        }
+        for (int i = 0; i < 8; ++i)
+            stage_entry(st, row * kStageLd + (tid >> 5) + 8 * i, raw.ok[i] && raw.v[i] != 0.0, raw.q[i],
+                        raw.n[i] - 1.0);
     }
 };
 
@@ -227,33 +233,31 @@ __device__ inline void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-__device__ inline unsigned bf16_bits(double integer_digit) {
-    // Integer digits |d| <= 2^14 and their 2^-8 multiples have <= 8 significant
-    // bits (a power of two times an integer below 2^8 in magnitude, or a power
-    // of two): the float and bf16 conversions are exact.
-    return __float_as_uint(static_cast<float>(integer_digit)) >> 16;
-}
-
-__device__ inline unsigned f16_bits(double digit) {
-    // The w digits are integers of at most 11 significant bits times a power of two
-    // (|A| <= 2048, 32 b, 4 c with |b|, |c| <= 1024, |D| <= 512) and V is 0 or 1: the
-    // float and FP16 conversions are exact.
-    return __builtin_bit_cast(unsigned short, static_cast<_Float16>(static_cast<float>(digit)));
+// Byte columns of four dwords: out[i] = byte i of x[0], x[1], x[2], x[3].
+__device__ inline void bytes4x4(const unsigned (&x)[4], unsigned (&out)[4]) {
+    const unsigned a01 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u);
+    const unsigned b01 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u);
+    const unsigned a23 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u);
+    const unsigned b23 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
 }
 
 template <class Src>
-__global__ __launch_bounds__(256) void prep_split_kernel(Src src, int P, int G32, int G16,
+__global__ __launch_bounds__(256) void prep_split_kernel(Src src, int P, int G32,
                                                          const std::int64_t* __restrict__ bt_s0,
                                                          const std::int32_t* __restrict__ bt_len,
                                                          const std::int64_t* __restrict__ bt_k0,
                                                          const std::int32_t* __restrict__ chunk_block,
-                                                         std::int64_t n_chunks, std::int64_t KS16,
-                                                         std::uint8_t* __restrict__ planes,
-                                                         i4* __restrict__ pV8) {
-    __shared__ double sq[32 * kStageLd];
-    __shared__ double sh[32 * kStageLd];
+                                                         std::int64_t n_chunks, std::int64_t KS32,
+                                                         std::uint8_t* __restrict__ planes) {
+    __shared__ Stage st;
     const int tid = threadIdx.x;
-    const int t4 = tid >> 6, lane = tid & 63;
+    // thread -> (q or w digits, 32-SNP step of the chunk, fragment lane)
+    const int lane = tid & 63, step = (tid >> 6) & 1;
+    const int set = __builtin_amdgcn_readfirstlane(tid >> 7);
     const std::int64_t n_units = static_cast<std::int64_t>(G32) * n_chunks;
     // Units run chunk-fastest so consecutive workgroups read adjacent row segments and
     // write adjacent plane chunks.  The next unit's inputs are fetched into registers
@@ -265,88 +269,43 @@ __global__ __launch_bounds__(256) void prep_split_kernel(Src src, int P, int G32
     std::int64_t u = blockIdx.x;
     if (u >= n_units) return;
     PrepUnit cur = prep_unit(u, n_chunks, bt_s0, bt_len, bt_k0, chunk_block);
-    src.put(src.fetch(32 * cur.g, P, cur.snp0, cur.live, tid), tid, sq, sh);
+    src.put(src.fetch(32 * cur.g, P, cur.snp0, cur.live, tid), tid, st);
     lds_barrier();
     for (;;) {
         const bool more = u + gridDim.x < n_units;
         const PrepUnit nxt = prep_unit(more ? u + gridDim.x : u, n_chunks, bt_s0, bt_len, bt_k0, chunk_block);
         const typename Src::Raw raw = src.fetch(32 * nxt.g, P, nxt.snp0, nxt.live, tid);
-        const int g = cur.g;
-        const std::int64_t c = cur.c;
 
-        // BF16 digit planes: thread -> (16-SNP step t4 of the chunk, fragment lane).
-        const int r = lane & 31;
-        unsigned w[kPlanes][4];
+        // Digit k of an integer is its byte 5 - k: digits 5..2 come from the low dword,
+        // digits 1 and 0 from this set's half of the shared one.
+        unsigned pl[kSetPlanes][4];
+        const unsigned* lo = set ? st.w : st.q;
+        const unsigned sel = set ? 0x07030602u : 0x05010400u;
 #pragma unroll
-        for (int p = 0; p < kPlanes; ++p)
+        for (int j4 = 0; j4 < 4; ++j4) {
+            const int at = (lane & 31) * kStageLd + 32 * step + 16 * (lane >> 5) + 4 * j4;
+            const unsigned x[4] = {lo[at], lo[at + 1], lo[at + 2], lo[at + 3]};
+            unsigned by[4];
+            bytes4x4(x, by);
 #pragma unroll
-            for (int hh = 0; hh < 4; ++hh) w[p][hh] = 0u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int kk = 16 * t4 + 8 * (lane >> 5) + j;
-            const double h = sh[r * kStageLd + kk];
-            if (h >= 0.0) {
-                double x = sq[r * kStageLd + kk] * 128.0;
-                double d[6];
-#pragma unroll
-                for (int k = 0; k < 6; ++k) {
-                    d[k] = rint(x);
-                    x = (x - d[k]) * 256.0;
-                }
-                const double qt =
-                    (d[0] + (d[1] + (d[2] + (d[3] + (d[4] + d[5] / 256.0) / 256.0) / 256.0) / 256.0) / 256.0) / 128.0;
-                // w in units of 2^-14, then the remainders in units of 2^-30 / 32, 2^-38 / 4
-                // and 2^-46 (every step is exact in FP64).
-                const double y = -0.5 * (qt * qt - h) * 16384.0;
-                const double wA = rint(y);
-                const double r1 = (y - wA) * 2048.0;
-                const double wb = rint(r1);
-                const double r2 = (r1 - wb) * 2048.0;
-                const double wc = rint(r2);
-                const double wD = rint((r2 - wc) * 1024.0);
-                const int sft = 16 * (j & 1);
-#pragma unroll
-                for (int k = 0; k < 5; ++k) w[k][j >> 1] |= bf16_bits(d[k]) << sft;
-                w[5][j >> 1] |= bf16_bits(d[5] / 256.0) << sft;
-                w[kPlaneA][j >> 1] |= f16_bits(wA) << sft;
-                w[kVPlane][j >> 1] |= f16_bits(1.0) << sft;
-                w[8][j >> 1] |= f16_bits(32.0 * wb) << sft;
-                w[9][j >> 1] |= f16_bits(4.0 * wc) << sft;
-                w[10][j >> 1] |= f16_bits(wD) << sft;
-            }
+            for (int i = 0; i < 4; ++i) pl[5 - i][j4] = by[i];
+            const unsigned t01 = __builtin_amdgcn_perm(st.t[at + 1], st.t[at], sel);
+            const unsigned t23 = __builtin_amdgcn_perm(st.t[at + 3], st.t[at + 2], sel);
+            pl[1][j4] = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
+            pl[0][j4] = __builtin_amdgcn_perm(t23, t01, 0x07060302u);
         }
-        // int8 V plane for the pair-count kernel (16x16x64 layout): the unit's two
-        // 16-row groups, one 16-byte fragment per thread of the first two wavefronts.
-        // Stored before the digit planes, so that the next unit's loads are followed by
-        // exactly the 11 plane stores of every wavefront.
-        if (tid < 128) {
-            const int g16 = 2 * g + (tid >> 6);
-            if (g16 < G16) {
-                const int rr = 16 * (tid >> 6) + (lane & 15);
-                const int kb = 16 * (lane >> 4);
-                unsigned v4[4] = {0, 0, 0, 0};
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    if (sh[rr * kStageLd + kb + j] >= 0.0) v4[j >> 2] |= 1u << (8 * (j & 3));
-                i4 v;
-                v[0] = static_cast<int>(v4[0]);
-                v[1] = static_cast<int>(v4[1]);
-                v[2] = static_cast<int>(v4[2]);
-                v[3] = static_cast<int>(v4[3]);
-                pV8[(static_cast<std::int64_t>(g16) * (KS16 / 4) + c) * 64 + lane] = v;
-            }
-        }
-        const std::int64_t t16 = 4 * c + t4;
-        std::uint8_t* base = planes + ((static_cast<std::int64_t>(g) * KS16 + t16) * kPlanes) * kChunk + lane * 16;
+        std::uint8_t* base =
+            planes + ((static_cast<std::int64_t>(cur.g) * KS32 + 2 * cur.c + step) * kPlanes + kSetPlanes * set) * kChunk +
+            lane * 16;
         // Streaming stores: the planes are far larger than the caches and are read back
         // by a later kernel in another order.
-        typedef unsigned u4v __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int p = 0; p < kPlanes; ++p)
-            __builtin_nontemporal_store(u4v{w[p][0], w[p][1], w[p][2], w[p][3]}, reinterpret_cast<u4v*>(base + p * kChunk));
+        for (int p = 0; p < kSetPlanes; ++p)
+            __builtin_nontemporal_store(u4v{pl[p][0], pl[p][1], pl[p][2], pl[p][3]},
+                                        reinterpret_cast<u4v*>(base + p * kChunk));
         if (!more) break;
         lds_barrier();  // every reader of this unit's stage is done
-        src.put(raw, tid, sq, sh);
+        src.put(raw, tid, st);
         lds_barrier();
         cur = nxt;
         u += gridDim.x;
@@ -355,16 +314,21 @@ __global__ __launch_bounds__(256) void prep_split_kernel(Src src, int P, int G32
 
 // ---------------------------------------------------------------------------------
 // pair counts: vpair_ij = sum_s v_i v_j by int8 MFMA (exact int32), written for both
-// (i,j) and (j,i).  Persistent 4-wavefront workgroups over (block, 128x128 tile pair)
-// items; wavefront w owns the 64x64 quadrant (rows 64 (w & 1), columns 64 (w >> 1)),
-// so every 16-row fragment a wavefront loads is loaded by one other wavefront of the
-// workgroup at the same time (the second load hits the CU's L1).  Quadrants below the
-// diagonal of a diagonal tile pair are skipped.
+// (i,j) and (j,i).  An entry is observed when bit 6 of its byte is set, in fragments of 32
+// rows x 32 SNPs `stride` bytes apart (the split form's W_0' plane, or the FP64 form's V
+// plane).  Persistent 4-wavefront workgroups over (block, 128x128 tile pair) items;
+// wavefront w owns the 64x64 quadrant (rows 64 (w & 1), columns 64 (w >> 1)), so every
+// fragment a wavefront loads is loaded by one other wavefront of the workgroup at the same
+// time (the second load hits the CU's L1).  Quadrants below the diagonal of a diagonal
+// tile pair are skipped.  Two K-steps are in flight while the two before them are
+// multiplied (blocks are padded to 64 SNPs, so steps come in pairs).
 // ---------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void count_kernel(const i4* __restrict__ pV8, BlockTable bt,
-                                                    const F2Item* __restrict__ items, ItemQueues queues,
-                                                    unsigned* __restrict__ counters, int P, int G16,
-                                                    std::int64_t KS64, double* __restrict__ vpair) {
+__device__ inline i4 observed(i4 x) { return (x >> 6) & 0x01010101; }
+
+__global__ __launch_bounds__(256) void count_kernel(const std::uint8_t* __restrict__ vplane, std::int64_t stride,
+                                                    BlockTable bt, const F2Item* __restrict__ items,
+                                                    ItemQueues queues, unsigned* __restrict__ counters, int P,
+                                                    int G32, std::int64_t KS32, double* __restrict__ vpair) {
     __shared__ int s_item;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -383,44 +347,71 @@ __global__ __launch_bounds__(256) void count_kernel(const i4* __restrict__ pV8, 
         const int ti = __builtin_amdgcn_readfirstlane(static_cast<int>(wi.ti));
         const int tj = __builtin_amdgcn_readfirstlane(static_cast<int>(wi.tj));
         if (ti == tj && rh > ch) continue;
-        const int gI0 = 8 * ti + 4 * rh;
-        const int gJ0 = 8 * tj + 4 * ch;
-        if (gI0 >= G16 || gJ0 >= G16) continue;
-        const std::int64_t u0 = bt.k0[b] / 64;
-        const int nu = bt.kpad[b] / 64;
-        bool rowI[4], rowJ[4];
+        const int gI0 = 4 * ti + 2 * rh;
+        const int gJ0 = 4 * tj + 2 * ch;
+        if (gI0 >= G32 || gJ0 >= G32) continue;
+        const std::int64_t t0 = bt.k0[b] / 32;
+        const int nsteps = __builtin_amdgcn_readfirstlane(bt.kpad[b] / 32);
+        // the second group of a pair past the last one re-reads the first (never written out)
+        const std::uint8_t* pI[2];
+        const std::uint8_t* pJ[2];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) { rowI[x] = gI0 + x < G16; rowJ[x] = gJ0 + x < G16; }
-        i4 cnt[4][4];
+        for (int x = 0; x < 2; ++x) {
+            pI[x] = vplane + (static_cast<std::int64_t>(gI0 + x < G32 ? gI0 + x : gI0) * KS32 + t0) * stride + lane * 16;
+            pJ[x] = vplane + (static_cast<std::int64_t>(gJ0 + x < G32 ? gJ0 + x : gJ0) * KS32 + t0) * stride + lane * 16;
+        }
+        i16v cnt[2][2];
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
+        for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int y = 0; y < 4; ++y) cnt[x][y] = i4{0, 0, 0, 0};
-        for (int u = 0; u < nu; ++u) {
-            i4 cI[4], cJ[4];
+            for (int y = 0; y < 2; ++y) cnt[x][y] = i16v{};
+        i4 cI[2][2], cJ[2][2];
+        auto load = [&](int t, i4 (&fI)[2][2], i4 (&fJ)[2][2]) {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                cI[x] = rowI[x] ? pV8[((gI0 + x) * KS64 + u0 + u) * 64 + lane] : i4{0, 0, 0, 0};
-                cJ[x] = rowJ[x] ? pV8[((gJ0 + x) * KS64 + u0 + u) * 64 + lane] : i4{0, 0, 0, 0};
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    fI[u][x] = *reinterpret_cast<const i4*>(pI[x] + (t + u) * stride);
+                    fJ[u][x] = *reinterpret_cast<const i4*>(pJ[x] + (t + u) * stride);
+                }
+        };
+        if (nsteps > 0) load(0, cI, cJ);
+        for (int t = 0; t < nsteps; t += 2) {
+            i4 nI[2][2], nJ[2][2];
+            load(t + 2 < nsteps ? t + 2 : t, nI, nJ);   // the last pair re-reads itself
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                i4 vI[2], vJ[2];
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    vI[x] = observed(cI[u][x]);
+                    vJ[x] = observed(cJ[u][x]);
+                }
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+                        cnt[x][y] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vI[x], vJ[y], cnt[x][y], 0, 0, 0);
             }
 #pragma unroll
-            for (int x = 0; x < 4; ++x)
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int y = 0; y < 4; ++y)
-                    if (rowI[x] && rowJ[y] && gI0 + x <= gJ0 + y)
-                        cnt[x][y] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cI[x], cJ[y], cnt[x][y], 0, 0, 0);
+                for (int x = 0; x < 2; ++x) {
+                    cI[u][x] = nI[u][x];
+                    cJ[u][x] = nJ[u][x];
+                }
         }
         double* vpb = vpair + slab * b;
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
+        for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int y = 0; y < 4; ++y) {
+            for (int y = 0; y < 2; ++y) {
                 const int gI = gI0 + x, gJ = gJ0 + y;
-                if (!(rowI[x] && rowJ[y] && gI <= gJ)) continue;
-                const int col = 16 * gJ + (lane & 15);
+                if (gI >= G32 || gJ >= G32 || gI > gJ) continue;
+                const int col = 32 * gJ + (lane & 31);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = 16 * gI + 4 * (lane >> 4) + e;
+                for (int e = 0; e < 16; ++e) {
+                    const int row = 32 * gI + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
                     if (row >= P || col >= P || (gI == gJ && row > col)) continue;
                     const double vp = static_cast<double>(cnt[x][y][e]);
                     vpb[row + static_cast<std::int64_t>(P) * col] = vp;
@@ -433,21 +424,15 @@ __global__ __launch_bounds__(256) void count_kernel(const i4* __restrict__ pV8, 
 // ---------------------------------------------------------------------------------
 // The split contraction.
 // ---------------------------------------------------------------------------------
-__device__ inline bf8 lds_frag(const std::uint8_t* slot, int group, int plane, int nplanes, int lane) {
-    return *reinterpret_cast<const bf8*>(slot + (group * nplanes + plane) * kChunk + lane * 16);
+__device__ inline i4 lds_frag(const std::uint8_t* slot, int group, int plane, int lane) {
+    return *reinterpret_cast<const i4*>(slot + (group * kSetPlanes + plane) * kChunk + lane * 16);
 }
 
-// Multiply 8 BF16 values by 2^-8 (exact: the values are small integers or zero).
-__device__ inline bf8 scale_2m8(bf8 a) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    u4 x = __builtin_bit_cast(u4, a);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float lo = __uint_as_float(x[i] << 16) * 0.00390625f;
-        const float hi = __uint_as_float(x[i] & 0xFFFF0000u) * 0.00390625f;
-        x[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-    }
-    return __builtin_bit_cast(bf8, x);
+// V = -128 v from W_0': bit 6 of each byte moved to its sign bit.
+__device__ inline i4 v_of_w0(i4 w0) {
+    u4v x = __builtin_bit_cast(u4v, w0);
+    x = (x << 1) & 0x80808080u;
+    return __builtin_bit_cast(i4, x);
 }
 
 // s_waitcnt on the vector-memory count only (gfx9 encoding: vmcnt in bits 3:0 and
@@ -459,250 +444,278 @@ __device__ inline void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// Slot kinds of a K-step: 0 = q digits d0..d5 (planes 0-5), 1 = X (A, V and, in RING 1,
-// B: planes 6-7 or 6-8), 2 = Y (the rest of B, C, D: planes 8-10 or 9-10).
-template <int kind, int RING>
-constexpr int slot_planes() {
-    return kind == 0 ? kDPlanes : (kind == 1 ? x_planes<RING>() : y_planes<RING>());
-}
-template <int kind, int RING>
-constexpr int slot_first_plane() {
-    return kind == 0 ? 0 : (kind == 1 ? kPlaneA : kPlaneA + x_planes<RING>());
+// Issue this wavefront's share of one slot's 1 KB chunks (direct global->LDS): chunk
+// ci = wave + 8 r from its source row `src[r]` (uniform) at byte `off` (per lane).
+// Every wavefront issues exactly kSetPlanes loads per slot, and chunk ci of a slot is
+// always loaded by wavefront ci % 8; the compile-time count lets the compiler's
+// wait-count tracking see how many loads follow each slot's, so that it adds no wait of
+// its own beyond the explicit ones.
+__device__ inline void stage_slot(const std::uint8_t* const (&src)[kSetPlanes], std::uint8_t* slot, unsigned off,
+                                  int wave) {
+#pragma unroll
+    for (int r = 0; r < kSetPlanes; ++r)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[r] + off),
+                                         (__attribute__((address_space(3))) void*)(slot + (wave + kWaves * r) * kChunk),
+                                         16, 0, 0);
 }
 
-// Issue this wavefront's share of one slot's 1 KB chunks (direct global->LDS).
-// Every wavefront issues exactly (8 groups * planes) / 8 = planes loads per slot, and
-// chunk ci of a slot is always loaded by wavefront ci % 8; the compile-time count
-// lets the compiler's wait-count tracking see how many loads follow each slot's, so
-// that it adds no wait of its own beyond the explicit ones.
-template <int kind, int RING>
-__device__ inline void stage_slot(const std::uint8_t* __restrict__ planes, std::uint8_t* slot, std::int64_t t16,
-                                  std::int64_t KS16, int gI0, int gJ0, int G32, int wave, int lane) {
-    constexpr int np = slot_planes<kind, RING>();
+// The products of one phase for the wavefront's NX sub-tiles: left groups li .. li + NX - 1
+// against right group rj of a slot.
+template <int NX>
+__device__ __forceinline__ void mul_q_c(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+    i4 dj[6];
 #pragma unroll
-    for (int r = 0; r < np; ++r) {
-        const int ci = wave + kWaves * r;
-        const int lg = ci / np, pp = ci - lg * np;
-        int gg = lg < 4 ? gI0 + lg : gJ0 + lg - 4;
-        if (gg >= G32) gg = 0;  // rows beyond P: any valid address; never read back
-        const std::uint8_t* src =
-            planes + ((static_cast<std::int64_t>(gg) * KS16 + t16) * kPlanes + slot_first_plane<kind, RING>() + pp) * kChunk +
-            lane * 16;
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src),
-                                         (__attribute__((address_space(3))) void*)(slot + ci * kChunk), 16, 0, 0);
+    for (int k = 0; k < 6; ++k) dj[k] = lds_frag(slot, rj, k, lane);
+    static_for<6>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+            const i4 di = lds_frag(slot, li + x, k, lane);
+#pragma unroll
+            for (int t = k; t < 6; ++t)
+                L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(di, dj[t - k], L[x][t], 0, 0, 0);
+        }
+    });
+}
+
+template <int NX>
+__device__ __forceinline__ void mul_w_c(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+    i4 wj[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) wj[k] = lds_frag(slot, rj, k, lane);
+    const i4 vj = v_of_w0(wj[0]);
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+        const i4 w0 = lds_frag(slot, li + x, 0, lane);
+        const i4 vi = v_of_w0(w0);
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            const i4 wt = t == 0 ? w0 : lds_frag(slot, li + x, t, lane);
+            L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wt, vj, L[x][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 6; ++t) L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vi, wj[t], L[x][t], 0, 0, 0);
     }
 }
 
-__device__ inline h8 lds_frag_h(const std::uint8_t* slot, int group, int plane, int nplanes, int lane) {
-    return *reinterpret_cast<const h8*>(slot + (group * nplanes + plane) * kChunk + lane * 16);
+// The same with each left fragment read from LDS one product group ahead of its use (the
+// compiler otherwise reads it right before).  The tuner chooses: 9.22 ms (compiler's order)
+// against 9.42 ms at 1000 populations x 600k SNPs, 1.27 against 1.32 ms at 200 x 1.2M.
+template <int NX>
+__device__ __forceinline__ void mul_q_a(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+    i4 dj[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) dj[k] = lds_frag(slot, rj, k, lane);
+    i4 di = lds_frag(slot, li, 0, lane);
+    static_for<6 * NX>([&](auto ic) {
+        constexpr int i = decltype(ic)::value, k = i / NX, x = i % NX;
+        constexpr int kn = (i + 1) / NX, xn = (i + 1) % NX;
+        i4 nx = di;
+        if constexpr (i + 1 < 6 * NX) nx = lds_frag(slot, li + xn, kn, lane);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = k; t < 6; ++t)
+            L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(di, dj[t - k], L[x][t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        di = nx;
+    });
 }
 
-template <int RING>
+template <int NX>
+__device__ __forceinline__ void mul_w_a(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+    i4 wj[6];
+    i4 wt = lds_frag(slot, li, 0, lane);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) wj[k] = lds_frag(slot, rj, k, lane);
+    const i4 vj = v_of_w0(wj[0]);
+    i4 vi{};
+    static_for<6 * NX>([&](auto ic) {
+        constexpr int i = decltype(ic)::value, x = i / 6, t = i % 6;
+        constexpr int xn = (i + 1) / 6, tn = (i + 1) % 6;
+        i4 nx = wt;
+        if constexpr (i + 1 < 6 * NX) nx = lds_frag(slot, li + xn, tn, lane);
+        if constexpr (t == 0) vi = v_of_w0(wt);
+        __builtin_amdgcn_sched_barrier(0);
+        L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wt, vj, L[x][t], 0, 0, 0);
+        L[x][(t + 3) % 6] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vi, wj[(t + 3) % 6], L[x][(t + 3) % 6], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        wt = nx;
+    });
+}
+
+// One work item as a wavefront sees it (every field uniform): a block's K range, the tile's
+// row groups, and the wavefront's NX sub-tiles, left groups gI .. gI + NX - 1 (li in the
+// slot) against right group gJ (rj in the slot).
+struct WaveItem {
+    std::int64_t t0;          // the block's first K-step
+    int b, nsteps;
+    int gI0, gJ0;             // the workgroup tile's first left and right row group
+    int gI, gJ, li, rj;
+};
+
+// Every wavefront of the workgroup runs the same number of barriers whatever its NX.
+template <int NX, bool kAhead>
+__device__ __forceinline__ void run_item(const WaveItem& wi, const std::uint8_t* __restrict__ planes,
+                                         std::int64_t KS32, int G32, int P, const double* __restrict__ vpair,
+                                         double* __restrict__ f2, const FixupList& fl, std::uint8_t* lds_0,
+                                         std::uint8_t* lds_1, std::uint8_t* lds_2, int wave, int lane) {
+    const int nsteps = wi.nsteps;
+    const std::int64_t slab = static_cast<std::int64_t>(P) * P;
+    for (int seg0 = 0;; seg0 += kSegSteps) {
+        const int seg_end = nsteps < seg0 + kSegSteps ? nsteps : seg0 + kSegSteps;
+        const bool last_seg = seg_end == nsteps;
+        const std::uint8_t* src[kSetPlanes];
+#pragma unroll
+        for (int r = 0; r < kSetPlanes; ++r) {
+            const int ci = wave + kWaves * r;
+            const int lg = ci / kSetPlanes, pp = ci - lg * kSetPlanes;
+            int gg = lg < 4 ? wi.gI0 + lg : wi.gJ0 + lg - 4;
+            if (gg >= G32) gg = 0;  // rows beyond P: any valid address; never read back
+            src[r] = planes + ((static_cast<std::int64_t>(gg) * KS32 + wi.t0 + seg0) * kPlanes + pp) * kChunk;
+        }
+        // Byte offset of plane set `set` of step s (look-ahead past the segment's end
+        // re-reads its last K-step, an empty block's prologue the step it was given; neither
+        // is read back).
+        auto offset = [&](int s, int set) {
+            const int k = s < seg_end ? s - seg0 : (seg_end > seg0 ? seg_end - 1 - seg0 : 0);
+            return static_cast<unsigned>((k * kPlanes + kSetPlanes * set) * kChunk + lane * 16);
+        };
+        i16v L[NX > 0 ? NX : 1][6];
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int t = 0; t < 6; ++t) L[x][t] = i16v{};
+
+        // Phase p = 2 step + set reads slot p % 3.  Per wavefront six loads per slot, all
+        // unconditional, so the explicit waits are exact on every path:
+        //   prologue:  D(0) -> slot 0, W(0) -> slot 1
+        //   phase p:   wait until at most six loads (phase p + 1's) are outstanding, so
+        //              this phase's have landed; barrier (every wavefront's have, and
+        //              every reader of phase p - 1's slot is done); issue phase p + 2
+        //              into that slot; multiply.
+        auto step_body = [&]<int r>(int step) {
+            std::uint8_t* const slots[3] = {lds_0, lds_1, lds_2};
+            constexpr int pd = (2 * r) % 3, pw = (2 * r + 1) % 3, pf = (2 * r + 2) % 3;
+            wait_vmcnt<kSetPlanes>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            stage_slot(src, slots[pf], offset(step + 1, 0), wave);
+            if constexpr (NX > 0 && kAhead) mul_q_a<NX>(L, slots[pd], wi.li, wi.rj, lane);
+            else if constexpr (NX > 0) mul_q_c<NX>(L, slots[pd], wi.li, wi.rj, lane);
+            wait_vmcnt<kSetPlanes>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            stage_slot(src, slots[pd], offset(step + 1, 1), wave);
+            if constexpr (NX > 0 && kAhead) mul_w_a<NX>(L, slots[pw], wi.li, wi.rj, lane);
+            else if constexpr (NX > 0) mul_w_c<NX>(L, slots[pw], wi.li, wi.rj, lane);
+        };
+        if (seg0 > 0) __syncthreads();  // every reader of the previous segment's slots is done
+        stage_slot(src, lds_0, offset(seg0, 0), wave);
+        stage_slot(src, lds_1, offset(seg0, 1), wave);
+        // The slot pattern repeats every three steps, so that each slot is a distinct LDS
+        // object in every access.
+        int step = seg0;
+        for (; step + 2 < seg_end; step += 3) {
+            step_body.template operator()<0>(step);
+            step_body.template operator()<1>(step + 1);
+            step_body.template operator()<2>(step + 2);
+        }
+        if (step < seg_end) step_body.template operator()<0>(step);
+        if (step + 1 < seg_end) step_body.template operator()<1>(step + 1);
+
+        // Epilogue: num = -2 sum_t U_t L_t; f2 = num / vpair.  The three upper and the
+        // three lower levels are combined exactly in 64-bit integers.  W_0's offset is
+        // taken back with the pairs counted up to each segment's end (for a segment before
+        // the last an integer share of them: the shares add up to the count).
+        double* f2b = f2 + slab * wi.b;
+        const double* vpb = vpair + slab * wi.b;
+        int el = lane;
+        asm volatile("" : "+v"(el));  // the output addresses are formed here, not kept through the K loop
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+            const int gI = wi.gI + x;
+            const int col = 32 * wi.gJ + (el & 31);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = 32 * gI + 8 * (e >> 2) + 4 * (el >> 5) + (e & 3);
+                const bool ok = row < P && col < P && !(gI == wi.gJ && row > col);
+                double val = 0.0, vp = 0.0;
+                if (ok) {
+                    const std::int64_t ij = row + static_cast<std::int64_t>(P) * col;
+                    vp = vpb[ij];
+                    int share = static_cast<int>(vp);
+                    if (seg0 > 0 || !last_seg) {
+                        const std::int64_t pairs = share;
+                        share = static_cast<int>(pairs * seg_end / nsteps) - static_cast<int>(pairs * seg0 / nsteps);
+                    }
+                    const std::int64_t l0 = L[x][0][e] + static_cast<std::int64_t>(kL0PerPair) * share;
+                    const std::int64_t hi = (l0 << 16) + (static_cast<std::int64_t>(L[x][1][e]) << 8) + L[x][2][e];
+                    const std::int64_t lo = (static_cast<std::int64_t>(L[x][3][e]) << 16) +
+                                            (static_cast<std::int64_t>(L[x][4][e]) << 8) + L[x][5][e];
+                    double num = -2.0 * (static_cast<double>(hi) * 0x1p-30 + static_cast<double>(lo) * 0x1p-54);
+                    if (seg0 > 0) num += f2b[ij];
+                    val = last_seg ? (vp > 0.0 ? num / vp : 0.0) : num;
+                    f2b[ij] = val;
+                    if (last_seg) f2b[col + static_cast<std::int64_t>(P) * row] = val;
+                }
+                if (last_seg) fixup_append(fl, ok && vp > 0.0 && fabs(val) < fl.tau, wi.b, row, col);
+            }
+        }
+        if (last_seg) break;
+    }
+}
+
+template <bool kAhead>
 __global__ __launch_bounds__(512) void f2_split_kernel(const std::uint8_t* __restrict__ planes, BlockTable bt,
                                                        const F2Item* __restrict__ items, ItemQueues queues,
                                                        unsigned* __restrict__ counters, int P, int G32,
-                                                       std::int64_t KS16, const double* __restrict__ vpair,
-                                                       double* __restrict__ f2, FixupList fl,
-                                                       int* __restrict__ item_slot) {
-    constexpr int kXPlanes = x_planes<RING>(), kYPlanes = y_planes<RING>();
-    constexpr int kXSlotBytes = kGroups * kXPlanes * kChunk, kYSlotBytes = kGroups * kYPlanes * kChunk;
+                                                       std::int64_t KS32, const double* __restrict__ vpair,
+                                                       double* __restrict__ f2, FixupList fl) {
     // One LDS object per ring slot: the compiler then knows that reads of one slot do
-    // not depend on the direct loads still landing in the others.  The q-digit slots
-    // and the A + V slots alternate between K-steps; B..D have one slot.
-    __shared__ __attribute__((aligned(16))) std::uint8_t lds_d0[kDSlotBytes];
-    __shared__ __attribute__((aligned(16))) std::uint8_t lds_d1[kDSlotBytes];
-    __shared__ __attribute__((aligned(16))) std::uint8_t lds_x0[kXSlotBytes];
-    __shared__ __attribute__((aligned(16))) std::uint8_t lds_x1[kXSlotBytes];
-    __shared__ __attribute__((aligned(16))) std::uint8_t lds_y[kYSlotBytes];
+    // not depend on the direct loads still landing in the others.
+    __shared__ __attribute__((aligned(16))) std::uint8_t lds_0[kSlotBytes];
+    __shared__ __attribute__((aligned(16))) std::uint8_t lds_1[kSlotBytes];
+    __shared__ __attribute__((aligned(16))) std::uint8_t lds_2[kSlotBytes];
+    __shared__ int s_item;
     const int lane = threadIdx.x & 63;
     // Wavefront-uniform values are moved to scalar registers so that every branch
     // on them is uniform and the MFMA accumulators never sit in divergent flow.
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int wa = wave & 1;   // left sub-tile: groups 2wa, 2wa+1 of the left tile
-    const int wc = wave >> 1;  // right sub-tile: group wc of the right tile
-    const std::int64_t slab = static_cast<std::int64_t>(P) * P;
-    const std::int64_t t_last = KS16 - 1;
 
     const int home = static_cast<int>(blockIdx.x % kXcds);
     int xq = 0;
     for (;;) {
-        int it;
-        if constexpr (RING == 0) {
-            __shared__ int s_item;
-            if (threadIdx.x == 0) s_item = claim_item(counters, queues, home, xq);
-            __syncthreads();
-            it = __builtin_amdgcn_readfirstlane(s_item);
-            __syncthreads();
-        } else {
-            if (threadIdx.x == 0)
-                __hip_atomic_store(&item_slot[blockIdx.x], claim_item(counters, queues, home, xq), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            __syncthreads();
-            it = __builtin_amdgcn_readfirstlane(
-                __hip_atomic_load(&item_slot[blockIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-            __syncthreads();
-        }
+        if (threadIdx.x == 0) s_item = claim_item(counters, queues, home, xq);
+        __syncthreads();
+        const int it = __builtin_amdgcn_readfirstlane(s_item);
+        __syncthreads();
         if (it < 0) break;
-        const F2Item wi = items[it];
-        const int b = __builtin_amdgcn_readfirstlane(wi.b);
-        const int gI0 = 4 * __builtin_amdgcn_readfirstlane(static_cast<int>(wi.ti));
-        const int gJ0 = 4 * __builtin_amdgcn_readfirstlane(static_cast<int>(wi.tj));
-        const std::int64_t t0 = bt.k0[b] / 16;
-        const int nsteps = __builtin_amdgcn_readfirstlane(bt.kpad[b] / 16);
-        // K-step index of step s, clamped: look-ahead loads past the block end (and the
-        // buffer end) re-read a valid K-step and are never read back.
-        auto kstep = [&](int s) { return t0 + s < t_last ? t0 + s : t_last; };
+        const F2Item f = items[it];
+        WaveItem wi;
+        wi.b = __builtin_amdgcn_readfirstlane(f.b);
+        wi.gI0 = 4 * __builtin_amdgcn_readfirstlane(static_cast<int>(f.ti));
+        wi.gJ0 = 4 * __builtin_amdgcn_readfirstlane(static_cast<int>(f.tj));
+        wi.t0 = bt.k0[wi.b] / 32;
+        if (wi.t0 >= KS32) wi.t0 = KS32 > 0 ? KS32 - 1 : 0;  // an empty last block: any valid step
+        wi.nsteps = __builtin_amdgcn_readfirstlane(bt.kpad[wi.b] / 32);
 
-        bool act[2];
+        // This wavefront's 32x32 sub-tiles: left groups li and li + 1, right group wc.
+        // Off the diagonal two row pairs x four columns.  A diagonal tile has the ten
+        // sub-tiles with li <= wc, dealt so that no SIMD (wavefronts w and w + 4) has more
+        // than three: (0,1) (1,1) | (0,2) (1,2) | (0,3) (1,3) | (2,3) (3,3) | (0,0) | (2,2).
+        const bool diag = wi.gI0 == wi.gJ0;
+        wi.li = diag ? 2 * ((0xE8 >> wave) & 1) : 2 * (wave & 1);
+        const int wc = diag ? (0x00203321 >> (4 * wave)) & 15 : wave >> 1;
+        wi.rj = 4 + wc;
+        wi.gI = wi.gI0 + wi.li;
+        wi.gJ = wi.gJ0 + wc;
+        int n_act = 0;
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const int li = 2 * wa + x;
-            act[x] = (gI0 + li < G32) && (gJ0 + wc < G32) && (gI0 < gJ0 || li <= wc);
-        }
-
-        f16v L[2][5], H[2];
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-#pragma unroll
-            for (int t = 0; t < 5; ++t) L[x][t] = f16v{};
-            H[x] = f16v{};
-        }
-
-        // Load schedule (per wavefront, loads per slot D 6, X 2 or 3, Y 3 or 2; all loads
-        // stage unconditionally, so every path issues the same counts and the explicit
-        // waits below are exact):
-        //   prologue:       D(0) -> d0, X(0) -> x0, D(1) -> d1
-        //   step s, phase d: wait until <= 6 + |X| loads are outstanding (D(s) done: only
-        //                    binding at s = 0), barrier (Y free), issue Y(s); q-digit
-        //                    products from D(s)
-        //   phase w:         wait for all (Y(s), and X(s), D(s+1) issued before it),
-        //                    barrier (D(s) and X(s-1) free), issue D(s+2) into D(s)'s
-        //                    slot and X(s+1) into X(s-1)'s; w-digit products from X(s), Y(s)
-        stage_slot<0, RING>(planes, lds_d0, kstep(0), KS16, gI0, gJ0, G32, wave, lane);
-        stage_slot<1, RING>(planes, lds_x0, kstep(0), KS16, gI0, gJ0, G32, wave, lane);
-        stage_slot<0, RING>(planes, lds_d1, kstep(1), KS16, gI0, gJ0, G32, wave, lane);
-
-        auto step_body = [&]<int par>(int step) {
-            std::uint8_t* const slot_d = par ? lds_d1 : lds_d0;
-            std::uint8_t* const slot_x = par ? lds_x1 : lds_x0;
-            std::uint8_t* const slot_xn = par ? lds_x0 : lds_x1;
-            // ---- q digits (BF16)
-            wait_vmcnt<kDPlanes + kXPlanes>();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            stage_slot<2, RING>(planes, lds_y, kstep(step), KS16, gI0, gJ0, G32, wave, lane);
-            {
-                bf8 dj[6];
-#pragma unroll
-                for (int k = 0; k < 6; ++k) dj[k] = lds_frag(slot_d, 4 + wc, k, kDPlanes, lane);
-                static_for<6>([&](auto kc) {
-                    constexpr int k = decltype(kc)::value;
-                    // Level 5 into L4: d5 is stored pre-scaled; for k = 1..4 the right
-                    // operand d_(5-k) is scaled here, once for both left sub-tiles (the
-                    // products are exact either way).
-                    const bf8 d5r = (k == 0 || k == 5) ? dj[5 - k] : scale_2m8(dj[5 - k]);
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) {
-                        if (!act[x]) continue;
-                        const bf8 di = lds_frag(slot_d, 2 * wa + x, k, kDPlanes, lane);
-#pragma unroll
-                        for (int t = k; t < 5; ++t)
-                            L[x][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(di, dj[t - k], L[x][t], 0, 0, 0);
-                        L[x][4] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(di, d5r, L[x][4], 0, 0, 0);
-                    }
-                });
-            }
-            // ---- w digits x V (FP16): A into L0, B, C, D into L2, L3, L4
-            wait_vmcnt<0>();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            stage_slot<0, RING>(planes, slot_d, kstep(step + 2), KS16, gI0, gJ0, G32, wave, lane);
-            stage_slot<1, RING>(planes, slot_xn, kstep(step + 1), KS16, gI0, gJ0, G32, wave, lane);
-            {
-                const h8 aj = lds_frag_h(slot_x, 4 + wc, 0, kXPlanes, lane);
-                const h8 vj = lds_frag_h(slot_x, 4 + wc, 1, kXPlanes, lane);
-                // w digits B, C, D: plane m of the three in X (after A, V) or Y
-                auto wfrag = [&](int group, int m) {
-                    return m < kXPlanes - 2 ? lds_frag_h(slot_x, group, 2 + m, kXPlanes, lane)
-                                            : lds_frag_h(lds_y, group, m - (kXPlanes - 2), kYPlanes, lane);
-                };
-                h8 wj[3];
-#pragma unroll
-                for (int m = 0; m < 3; ++m) wj[m] = wfrag(4 + wc, m);
-#pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    if (!act[x]) continue;
-                    const h8 ai = lds_frag_h(slot_x, 2 * wa + x, 0, kXPlanes, lane);
-                    const h8 vi = lds_frag_h(slot_x, 2 * wa + x, 1, kXPlanes, lane);
-                    L[x][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ai, vj, L[x][0], 0, 0, 0);
-                    L[x][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vi, aj, L[x][0], 0, 0, 0);
-#pragma unroll
-                    for (int m = 0; m < 3; ++m) {
-                        const h8 wi = wfrag(2 * wa + x, m);
-                        L[x][2 + m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wi, vj, L[x][2 + m], 0, 0, 0);
-                        L[x][2 + m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vi, wj[m], L[x][2 + m], 0, 0, 0);
-                    }
-                }
-                // Every 8 K-steps (128 SNPs) and at the block end: exact carries.
-                if ((step & 7) == 7 || step + 1 == nsteps) {
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) {
-                        if (!act[x]) continue;
-#pragma unroll
-                        for (int e = 0; e < 16; ++e) {
-#pragma unroll
-                            for (int t = 4; t >= 1; --t) {
-                                const float cr = rintf(L[x][t][e] * (1.0f / 256.0f));
-                                L[x][t][e] = fmaf(cr, -256.0f, L[x][t][e]);
-                                L[x][t - 1][e] += cr;
-                            }
-                            const float c0 = rintf(L[x][0][e] * (1.0f / 4096.0f)) * 4096.0f;
-                            L[x][0][e] -= c0;
-                            H[x][e] += c0;
-                        }
-                    }
-                }
-            }
-        };
-        // Steps alternate between the two q-digit (and A + V) slots; unrolled by two so
-        // that each slot is a distinct LDS object in every access, with an odd last step
-        // after the loop (so that both bodies always run inside it).
-        int step = 0;
-        for (; step + 1 < nsteps; step += 2) {
-            step_body.template operator()<0>(step);
-            step_body.template operator()<1>(step + 1);
-        }
-        if (step < nsteps) step_body.template operator()<0>(step);
-
-        // Epilogue: num = -2 sum_t U_t L_t in FP64; f2 = num / vpair.
-        double* f2b = f2 + slab * b;
-        const double* vpb = vpair + slab * b;
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            if (!act[x]) continue;
-            const int gI = gI0 + 2 * wa + x, gJ = gJ0 + wc;
-            const int col = 32 * gJ + (lane & 31);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = 32 * gI + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                const bool ok = row < P && col < P && !(gI == gJ && row > col);
-                double val = 0.0, vp = 0.0;
-                if (ok) {
-                    const double s = (static_cast<double>(H[x][e]) + static_cast<double>(L[x][0][e])) * 0x1p-14 +
-                                     static_cast<double>(L[x][1][e]) * 0x1p-22 +
-                                     static_cast<double>(L[x][2][e]) * 0x1p-30 +
-                                     static_cast<double>(L[x][3][e]) * 0x1p-38 +
-                                     static_cast<double>(L[x][4][e]) * 0x1p-46;
-                    const double num = -2.0 * s;
-                    const std::int64_t ij = row + static_cast<std::int64_t>(P) * col;
-                    vp = vpb[ij];
-                    val = vp > 0.0 ? num / vp : 0.0;
-                    f2b[ij] = val;
-                    f2b[col + static_cast<std::int64_t>(P) * row] = val;
-                }
-                fixup_append(fl, ok && vp > 0.0 && fabs(val) < fl.tau, b, row, col);
-            }
-        }
+        for (int x = 0; x < 2; ++x)
+            n_act += wi.gI + x < G32 && wi.gJ < G32 && (!diag || wi.li + x <= wc);
+        if (n_act == 2) run_item<2, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
+        else if (n_act == 1) run_item<1, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
+        else run_item<0, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
     }
     // The last item's look-ahead loads may still be landing in LDS: drain them before
     // the workgroup's LDS can be handed to another workgroup.
@@ -718,46 +731,53 @@ static unsigned prep_grid(std::int64_t n_units) {
 }
 
 void launch_prep_split_counts(const std::uint16_t* a2, const std::uint16_t* n, std::int64_t ld, int P, int G32,
-                              int G16, BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks,
-                              std::int64_t KS16, std::uint8_t* planes, void* pV8, hipStream_t st) {
+                              BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks,
+                              std::int64_t KS32, std::uint8_t* planes, hipStream_t st) {
     if (n_chunks <= 0 || G32 <= 0) return;
     prep_split_kernel<CountsSrc><<<prep_grid(G32 * n_chunks), 256, 0, st>>>(
-        CountsSrc{a2, n, ld}, P, G32, G16, bt.s0, bt.len, bt.k0, chunk_block, n_chunks, KS16, planes,
-        static_cast<i4*>(pV8));
+        CountsSrc{a2, n, ld}, P, G32, bt.s0, bt.len, bt.k0, chunk_block, n_chunks, KS32, planes);
     STP_LAUNCH_CHECK();
 }
 
-void launch_prep_split_qvn(const double* q, const double* v, const double* n, int P, int G32, int G16,
-                           BlockTable bt, const std::int32_t* chunk_block, std::int64_t n_chunks, std::int64_t KS16,
-                           std::uint8_t* planes, void* pV8, hipStream_t st) {
+void launch_prep_split_qvn(const double* q, const double* v, const double* n, int P, int G32, BlockTable bt,
+                           const std::int32_t* chunk_block, std::int64_t n_chunks, std::int64_t KS32,
+                           std::uint8_t* planes, hipStream_t st) {
     if (n_chunks <= 0 || G32 <= 0) return;
     prep_split_kernel<QvnSrc><<<prep_grid(G32 * n_chunks), 256, 0, st>>>(
-        QvnSrc{q, v, n}, P, G32, G16, bt.s0, bt.len, bt.k0, chunk_block, n_chunks, KS16, planes,
-        static_cast<i4*>(pV8));
+        QvnSrc{q, v, n}, P, G32, bt.s0, bt.len, bt.k0, chunk_block, n_chunks, KS32, planes);
     STP_LAUNCH_CHECK();
 }
 
-void launch_count(const void* pV8, BlockTable bt, const F2Item* items, const ItemQueues& queues,
-                  unsigned* counters, int P, int G16, std::int64_t KS64, double* vpair, int n_workgroups,
-                  hipStream_t st) {
+void launch_count_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
+                        unsigned* counters, int P, int G32, std::int64_t KS32, double* vpair, int n_workgroups,
+                        hipStream_t st) {
     if (queues.off[kXcds] <= 0) return;
     launch_zero_u32(counters, kXcds, st);
-    count_kernel<<<static_cast<unsigned>(n_workgroups), 256, 0, st>>>(static_cast<const i4*>(pV8), bt, items,
-                                                                      queues, counters, P, G16, KS64, vpair);
+    count_kernel<<<static_cast<unsigned>(n_workgroups), 256, 0, st>>>(
+        planes + kSetPlanes * kChunk, kPlanes * kChunk, bt, items, queues, counters, P, G32, KS32, vpair);
+    STP_LAUNCH_CHECK();
+}
+
+void launch_count_v8(const std::uint8_t* v8, BlockTable bt, const F2Item* items, const ItemQueues& queues,
+                     unsigned* counters, int P, int G32, std::int64_t KS32, double* vpair, int n_workgroups,
+                     hipStream_t st) {
+    if (queues.off[kXcds] <= 0) return;
+    launch_zero_u32(counters, kXcds, st);
+    count_kernel<<<static_cast<unsigned>(n_workgroups), 256, 0, st>>>(v8, kChunk, bt, items, queues, counters, P, G32,
+                                                                      KS32, vpair);
     STP_LAUNCH_CHECK();
 }
 
 void launch_f2_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
-                     unsigned* counters, int P, int G32, std::int64_t KS16, const double* vpair, double* f2,
-                     const FixupList& fl, int n_workgroups, int ring, int* item_slot, hipStream_t st) {
+                     unsigned* counters, int P, int G32, std::int64_t KS32, const double* vpair, double* f2,
+                     const FixupList& fl, int n_workgroups, int ring, hipStream_t st) {
     if (queues.off[kXcds] <= 0) return;
     launch_zero_u32(counters, kXcds, st);
+    const dim3 grid(static_cast<unsigned>(n_workgroups));
     if (ring == 1)
-        f2_split_kernel<1><<<static_cast<unsigned>(n_workgroups), 512, 0, st>>>(planes, bt, items, queues, counters, P,
-                                                                               G32, KS16, vpair, f2, fl, item_slot);
+        f2_split_kernel<true><<<grid, 512, 0, st>>>(planes, bt, items, queues, counters, P, G32, KS32, vpair, f2, fl);
     else
-        f2_split_kernel<0><<<static_cast<unsigned>(n_workgroups), 512, 0, st>>>(planes, bt, items, queues, counters, P,
-                                                                               G32, KS16, vpair, f2, fl, item_slot);
+        f2_split_kernel<false><<<grid, 512, 0, st>>>(planes, bt, items, queues, counters, P, G32, KS32, vpair, f2, fl);
     STP_LAUNCH_CHECK();
 }
 
