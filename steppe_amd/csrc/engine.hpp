@@ -501,11 +501,12 @@ private:
     bool timing_ = false;
     // qpAdm working set (grow-only): survivor-transposed f2, survivor sizes and list,
     // the model arena, per-workgroup scratch and the device result records.
-    DevBuf<double> qpT_, qp_scratch_;
+    DevBuf<double> qpT_;
     DevBuf<std::int32_t> qp_i32_, qp_keep_;
     DevBuf<stp_qpadm_result> qp_out_;
     // Large-model qpAdm working set (grow-only): model and task lists, fit tables,
     // per-model setup scratch, per-wavefront fit scratch, leave-one-block-out weights.
+    void qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, const stp_qpadm_options& opt);
     void qpadm_large(QpLargeArgs a, const std::vector<QpLargeModel>& large, int rank_opt);
     DevBuf<QpLargeModel> ql_models_;
     DevBuf<QpLargeTask> ql_tasks_;

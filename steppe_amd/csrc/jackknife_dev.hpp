@@ -82,6 +82,10 @@ __device__ bool wg_lu_inverse(double* lu, int ld, int m, double* inv, int ldi, i
     return true;
 }
 
+// The sums over the blocks run across the lanes of a wavefront and meet in a double-double
+// tree: with one thread per statistic and one per entry of Q they were chains of nbs
+// dependent double-double steps on uncoalesced loads.
+//
 // Workgroup-level; every thread of the workgroup calls it.  X [m][nbs] holds the
 // statistic per surviving block (global) and is overwritten by tau; LOO [m][nbs]
 // (global) receives the leave-one-out values.  Outputs: s_xtot / s_totline (m, LDS),
@@ -98,56 +102,63 @@ __device__ bool jk_covariance(double* X, double* LOO, const std::int32_t* bsz, d
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // ---- LOO and total (one thread per statistic) ----
-    for (int k = tid; k < m; k += kThreads) {
-        const double* Xk = X + static_cast<std::int64_t>(k) * nbs;
+    // ---- LOO, total and tau (one wavefront per statistic, lanes over the blocks) ----
+    for (int k = wave; k < m; k += kWaves) {
+        double* Xk = X + static_cast<std::int64_t>(k) * nbs;
         double* Lk = LOO + static_cast<std::int64_t>(k) * nbs;
         dd s{0.0, 0.0};
-        for (int b = 0; b < nbs; ++b) s = dd_fma(s, Xk[b], static_cast<double>(bsz[b]));
-        const double tot = dd_div_d(s, n_tot);
-        for (int b = 0; b < nbs; ++b) {
-            const double rel = static_cast<double>(bsz[b]) / n_tot;
-            Lk[b] = (tot - Xk[b] * rel) / (1.0 - rel);
-        }
-        dd wn{0.0, 0.0}, wd{0.0, 0.0};
-        for (int b = 0; b < nbs; ++b) {
-            const double w = 1.0 - static_cast<double>(bsz[b]) / n_tot;
-            wn = dd_fma(wn, Lk[b], w);
+        for (int b = lane; b < nbs; b += 64) s = dd_fma(s, Xk[b], static_cast<double>(bsz[b]));
+        const double tot = dd_div_d(wave_total_dd(s), n_tot);
+        dd wn{0.0, 0.0}, wd{0.0, 0.0}, wb{0.0, 0.0};
+        for (int b = lane; b < nbs; b += 64) {
+            const double sz = static_cast<double>(bsz[b]);
+            const double rel = sz / n_tot, w = 1.0 - rel;
+            const double l = (tot - Xk[b] * rel) / w;
+            Lk[b] = l;
+            wn = dd_fma(wn, l, w);
             wd = dd_add(wd, w);
+            wb = dd_fma(wb, l, sz);
         }
-        const double tl = dd_div_dd(wn, wd);
+        const double tl = dd_div_dd(wave_total_dd(wn), wave_total_dd(wd));
+        wb = wave_total_dd(wb);
         dd ds{0.0, 0.0};
-        for (int b = 0; b < nbs; ++b) ds = dd_add(dd_add(ds, tl), -Lk[b]);
-        const double term1 = dd_div_d(ds, static_cast<double>(nbs)) * static_cast<double>(nbs);
-        dd wb{0.0, 0.0};
-        for (int b = 0; b < nbs; ++b) wb = dd_fma(wb, Lk[b], static_cast<double>(bsz[b]));
-        s_totline[k] = tl;
-        s_xtot[k] = term1 + dd_div_d(wb, n_tot);
-    }
-    __syncthreads();
-    // ---- tau, overwriting X ----
-    for (int k = wave; k < m; k += kWaves) {
-        const double xt = s_xtot[k], tl = s_totline[k];
+        for (int b = lane; b < nbs; b += 64) ds = dd_add(dd_add(ds, tl), -Lk[b]);
+        const double term1 = dd_div_d(wave_total_dd(ds), static_cast<double>(nbs)) * static_cast<double>(nbs);
+        const double xt = term1 + dd_div_d(wb, n_tot);
+        if (lane == 0) {
+            s_totline[k] = tl;
+            s_xtot[k] = xt;
+        }
         for (int b = lane; b < nbs; b += 64) {
             const double h = n_tot / static_cast<double>(bsz[b]);
-            const double sq = sqrt(h - 1.0);
-            const std::int64_t o = static_cast<std::int64_t>(k) * nbs + b;
-            X[o] = (xt * h - LOO[o] * (h - 1.0) - tl) / sq;
+            Xk[b] = (xt * h - Lk[b] * (h - 1.0) - tl) / sqrt(h - 1.0);
         }
     }
     __syncthreads();
-    // ---- Q = sum_b tau tau^T / nb (upper triangle, mirrored) into sLU ----
-    for (int e = tid; e < m * m; e += kThreads) {
-        const int a = e / m, c = e - (e / m) * m;
-        if (c < a) continue;
-        const double* ta = X + static_cast<std::int64_t>(a) * nbs;
-        const double* tc = X + static_cast<std::int64_t>(c) * nbs;
-        dd acc{0.0, 0.0};
-        for (int b = 0; b < nbs; ++b) acc = dd_fma(acc, ta[b], tc[b]);
-        const double v = dd_div_d(acc, static_cast<double>(nbs));
-        sLU[a * ldq + c] = v;
-        sLU[c * ldq + a] = v;
-    }
+    // ---- Q = sum_b tau tau^T / nb (upper triangle, mirrored) into sLU: a wavefront takes
+    // four entries of a row at a time, lanes over the blocks ----
+    int turn = 0;
+    for (int a = 0; a < m; ++a)
+        for (int c0 = a; c0 < m; c0 += 4) {
+            if (turn++ % kWaves != wave) continue;
+            const double* ta = X + static_cast<std::int64_t>(a) * nbs;
+            const double* tc[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tc[i] = X + static_cast<std::int64_t>(min(c0 + i, m - 1)) * nbs;
+            dd acc[4] = {};
+            for (int b = lane; b < nbs; b += 64) {
+                const double t = ta[b];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = dd_fma(acc[i], t, tc[i][b]);
+            }
+            const dd q = wave_total4_dd(acc);
+            const int c = c0 + (lane >> 2);
+            if (lane < 16 && (lane & 3) == 0 && c < m) {
+                const double v = dd_div_d(q, static_cast<double>(nbs));
+                sLU[static_cast<std::int64_t>(a) * ldq + c] = v;
+                sLU[static_cast<std::int64_t>(c) * ldq + a] = v;
+            }
+        }
     __syncthreads();
     if (tid == 0) {
         double tr = 0.0;

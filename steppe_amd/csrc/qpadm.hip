@@ -1,8 +1,9 @@
 // steppe_amd/csrc/qpadm.hip — batched qpAdm fits on the device-resident f2 tensor.
 //
-// One workgroup (4 wavefronts) fits one model at a time and loops over the models of
-// its launch (a shared atomic cursor hands them out in decreasing-cost order).  Per
-// model it runs the reference's fit chain (src/core/qpadm/qpadm_fit.cpp:49-132):
+// A call's models go through four launches: setup (a workgroup per model: f4 basis, LOO,
+// covariance), the fit table (a workgroup per model, a wavefront per fit), the refits (most
+// shapes in qpadm_rows.hip, the others here) and the record.  Per model that is the
+// reference's fit chain (src/core/qpadm/qpadm_fit.cpp:49-132):
 //
 //   f4 basis        X[k][b] = (f2(Li,R0) + f2(L0,Rj) - f2(L0,R0) - f2(Li,Rj)) / 2,
 //                   k = j + nr*i, over the surviving blocks
@@ -393,106 +394,109 @@ constexpr int qpadm_waves_per_simd() {
     return T == 16 ? 5 : (T == 32 ? 4 : (T == 48 ? 3 : 1));
 }
 
-template <int T>
-__global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(qpadm_waves_per_simd<T>())))
-void qpadm_kernel(QpadmArgs g) {
+// Per-wave LDS slices of the fits, after `used` doubles of the workgroup's.
+__device__ inline int wave_slice(int nr_max) { return 416 + nr_max * nr_max + (kMaxQpadmNr + 1) / 2 + 1; }
+__device__ inline WaveSlice slice_at(double* p, int nr_max) {
+    WaveSlice W;
+    W.x = p;
+    W.y = p + 64;
+    W.a = p + 128;
+    W.b = p + 192;
+    W.w = p + 256;
+    W.ws = p + 320;
+    W.sig = p + 384;
+    W.v = p + 416;
+    W.ord = reinterpret_cast<int*>(p + 416 + nr_max * nr_max);
+    return W;
+}
+
+// One model per workgroup: f4 basis, leave-one-out values and total, jackknife covariance and
+// its inverse.
+__global__ __launch_bounds__(kQThreads) void qpadm_setup_kernel(QpFitArgs g) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
-    __shared__ int s_model, s_status, s_next, s_nfit;
+    __shared__ int s_status;
     __shared__ int s_L[kMaxNl + 1];
     __shared__ int s_R[kMaxQpadmNr + 1];
     __shared__ int s_pos[kMaxQpadmM], s_lane_of[2 * kQWaves + 2];
     __shared__ double s_val[kQWaves + 1];
-    __shared__ signed char s_fit_row[kMaxRows * kMaxRanks + 2], s_fit_rank[kMaxRows * kMaxRanks + 2];
-    __shared__ double s_chisq[kMaxRows][kMaxRanks];
-    __shared__ double s_wrf[kMaxRows][kMaxNl];  // weights of each popdrop row's fit at rank nlr-1
-    __shared__ double s_wmain[kMaxNl];          // weights of the main fit when its rank differs
-    __shared__ int s_ok[kMaxRows][kMaxRanks];
     __shared__ double s_xtot[kMaxQpadmM], s_totline[kMaxQpadmM];
-    __shared__ double s_prank[kMaxRanks];
-
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ldq = g.ldq;
-    double* const sQi = lds;                                   // Qinv, m x ldq
-    double* const sLU = lds + g.m_max * ldq;                   // Qf / its LU (setup only)
-    double* const wbase = sLU;                                 // per-wave slices (fit phase)
-    const int wstride = g.wave_slice;
-    WaveSlice W;
+    const QpLargeModel md = g.models[blockIdx.x];
+    const int nl = md.nl, nr = md.nr, m = md.m, nbs = g.nbs, ldq = m + 1;
+    double* const sQi = lds;
+    double* const sLU = lds + m * ldq;
+    if (tid == 0) s_L[0] = g.target[md.mi];
+    if (tid < nl) s_L[tid + 1] = g.left[md.l0 + tid];
+    if (tid <= nr) s_R[tid] = g.right[md.r0 + tid];
+    __syncthreads();
+    const QpSetup sp = qp_setup(g.setup, md, nbs);
     {
-        double* p = wbase + wave * wstride;
-        W.x = p;
-        W.y = p + 64;
-        W.a = p + 128;
-        W.b = p + 192;
-        W.w = p + 256;
-        W.ws = p + 320;
-        W.sig = p + 384;
-        W.v = p + 416;
-        W.ord = reinterpret_cast<int*>(p + 416 + g.nr_max * g.nr_max);
+        const int P = g.P;
+        const std::int64_t ld2 = nbs;
+        const int L0 = s_L[0], R0 = s_R[0];
+        const double* f00 = g.f2T + (L0 + static_cast<std::int64_t>(P) * R0) * ld2;
+        for (int k = wave; k < m; k += kQWaves) {
+            const int i = k / nr, j = k - (k / nr) * nr;
+            const int Li = s_L[i + 1], Rj = s_R[j + 1];
+            const double* fi0 = g.f2T + (Li + static_cast<std::int64_t>(P) * R0) * ld2;
+            const double* f0j = g.f2T + (L0 + static_cast<std::int64_t>(P) * Rj) * ld2;
+            const double* fij = g.f2T + (Li + static_cast<std::int64_t>(P) * Rj) * ld2;
+            for (int b = lane; b < nbs; b += 64)
+                sp.X[static_cast<std::int64_t>(k) * nbs + b] = 0.5 * (fi0[b] + f0j[b] - f00[b] - fij[b]);
+        }
     }
-    double* const scr = g.scratch + static_cast<std::int64_t>(blockIdx.x) * g.scratch_stride;
-    const int nbs = g.nbs;
-    double* const sX = scr;                                    // X, then tau: [m][nbs]
-    double* const sLOO = scr + static_cast<std::int64_t>(g.m_max) * nbs;      // [m][nbs]
-    double* const sWM = sLOO + static_cast<std::int64_t>(g.m_max) * nbs;      // [nbs][nl]
-    const double n_tot = g.n_total;
-
-    for (;;) {
-        if (tid == 0) s_model = static_cast<int>(atomicAdd(g.counter, 1u));
-        __syncthreads();
-        const int slot = __builtin_amdgcn_readfirstlane(s_model);
-        __syncthreads();
-        if (slot >= g.n_order) break;
-        const int mi = g.order[slot];
-        const int l0 = g.left_off[mi], l1 = g.left_off[mi + 1];
-        const int r0 = g.right_off[mi], r1 = g.right_off[mi + 1];
-        const int nl = l1 - l0, nr = r1 - r0 - 1, m = nl * nr;
-        const int rank = g.rank < 0 ? nl - 1 : g.rank;
-        if (tid == 0) s_L[0] = g.target[mi];
-        if (tid < nl) s_L[tid + 1] = g.left[l0 + tid];
-        if (tid <= nr) s_R[tid] = g.right[r0 + tid];
-        __syncthreads();
-        stp_qpadm_result* out = g.out + mi;
-
-        // ---- f4 basis over the surviving blocks ----
-        {
-            const int P = g.P;
-            const std::int64_t ld2 = nbs;
-            const int L0 = s_L[0], R0 = s_R[0];
-            const double* f00 = g.f2T + (L0 + static_cast<std::int64_t>(P) * R0) * ld2;
-            for (int k = wave; k < m; k += kQWaves) {
-                const int i = k / nr, j = k - (k / nr) * nr;
-                const int Li = s_L[i + 1], Rj = s_R[j + 1];
-                const double* fi0 = g.f2T + (Li + static_cast<std::int64_t>(P) * R0) * ld2;
-                const double* f0j = g.f2T + (L0 + static_cast<std::int64_t>(P) * Rj) * ld2;
-                const double* fij = g.f2T + (Li + static_cast<std::int64_t>(P) * Rj) * ld2;
-                for (int b = lane; b < nbs; b += 64)
-                    sX[static_cast<std::int64_t>(k) * nbs + b] = 0.5 * (fi0[b] + f0j[b] - f00[b] - fij[b]);
-            }
+    __syncthreads();
+    const bool ok = jk_covariance<kQThreads>(sp.X, sp.LOO, g.bsz, g.n_total, nbs, m, g.fudge, s_xtot, s_totline,
+                                             nullptr, sLU, ldq, sQi, ldq, s_pos, s_lane_of, s_val, &s_status);
+    if (ok) {
+        for (int e = tid; e < m * m; e += kQThreads) {
+            const int a = e / m;
+            sp.Qi[e] = sQi[a * ldq + (e - a * m)];
         }
-        __syncthreads();
-        // ---- LOO / total, jackknife covariance, ridge and its inverse ----
-        const bool cov_ok = jk_covariance<kQThreads>(sX, sLOO, g.bsz, n_tot, nbs, m, g.fudge, s_xtot, s_totline,
-                                                     nullptr, sLU, ldq, sQi, ldq, s_pos, s_lane_of, s_val,
-                                                     &s_status);
-        if (!cov_ok) {
-            if (tid == 0) {
-                out->status = 3;  // NonSpdCovariance
-                out->model_index = mi;
-                out->nl = 0;
-                out->est_rank = rank;
-                out->dof = dof_of(nl, nr, rank);
-                out->n_rank = 0;
-                out->n_popdrop = 0;
-            }
-            continue;
+        if (tid < m) {
+            sp.xtot[tid] = s_xtot[tid];
+            sp.totline[tid] = s_totline[tid];
         }
+    }
+    if (tid == 0) g.tables[blockIdx.x].cov_ok = ok ? 1 : 0;
+}
 
-        // ---- fit table: rank sweeps of the full model and of each popdrop row ----
-        const int nrows = nl >= 2 ? nl + 1 : 1;
-        if (tid == 0) {
-            int n = 0;
+// The fits of a model with a wavefront per fit: workgroup (part, model).  Without refits one
+// part per model runs its fit table (rank sweeps of the full model and of each popdrop row);
+// with refits part p takes kRefitPart leave-one-block-out refits.
+constexpr int kRefitPart = 32;
+
+template <int T>
+__global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(qpadm_waves_per_simd<T>())))
+void qpadm_fit_kernel(QpFitArgs g, int n_parts, int refits, int nr_max) {
+    extern __shared__ __attribute__((aligned(16))) double lds[];
+    __shared__ int s_next, s_nfit;
+    __shared__ signed char s_fit_row[kMaxRows * kMaxRanks + 2], s_fit_rank[kMaxRows * kMaxRanks + 2];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slot = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / n_parts);
+    const int part = static_cast<int>(blockIdx.x) - slot * n_parts;
+    const QpLargeModel md = g.models[slot];
+    QpLargeTables* tb = g.tables + slot;
+    if (!tb->cov_ok) return;
+    const int nl = md.nl, nr = md.nr, m = md.m, nbs = g.nbs, rank = md.rank, ldq = m + 1;
+    const QpSetup sp = qp_setup(g.setup, md, nbs);
+    const double* wmain = rank == nl - 1 ? tb->wrf[0] : tb->wmain;
+    if (refits && !qpadm_do_se(tb->ok[0][rank] != 0, nbs, g.jackknife, wmain, nl, g.se_require_p != 0,
+                               tb->chisq[0][rank], dof_of(nl, nr, rank), g.p_se_threshold))
+        return;
+    const WaveSlice W = slice_at(lds + m * ldq + wave * wave_slice(nr_max), nr_max);
+    for (int e = tid; e < m * m; e += kQThreads) {
+        const int a = e / m;
+        lds[a * ldq + (e - a * m)] = sp.Qi[e];
+    }
+    if (tid == 0) {
+        int n = 0;
+        if (!refits) {
+            const int nrows = nl >= 2 ? nl + 1 : 1;
             for (int k = 0; k < nrows; ++k) {
                 const int nlr = k == 0 ? nl : nl - 1;
                 const int rmax = min(nlr, nr) - 1, rf = nlr - 1;
@@ -509,72 +513,79 @@ void qpadm_kernel(QpadmArgs g) {
                     s_fit_rank[n++] = static_cast<signed char>(rank);
                 }
             }
-            s_nfit = n;
-            s_next = 0;
         }
-        __syncthreads();
-        for (;;) {
-            int f = 0;
-            if (lane == 0) f = atomicAdd(&s_next, 1);
-            f = __builtin_amdgcn_readfirstlane(__shfl(f, 0));
-            if (f >= s_nfit) break;
+        s_nfit = refits ? min(nbs, (part + 1) * kRefitPart) : n;
+        s_next = refits ? part * kRefitPart : 0;
+    }
+    __syncthreads();
+    const int n_fit = __builtin_amdgcn_readfirstlane(s_nfit);
+    for (;;) {
+        int f = 0;
+        if (lane == 0) f = atomicAdd(&s_next, 1);
+        f = __builtin_amdgcn_readfirstlane(__shfl(f, 0));
+        if (f >= n_fit) break;
+        double chisq = 0.0;
+        if (refits) {
+            if (lane < m) W.x[lane] = sp.LOO[static_cast<std::int64_t>(lane) * nbs + f];
+            __builtin_amdgcn_wave_barrier();
+            double* wrow = W.sig;  // nl weights; sig is free after the seed
+            const bool ok = als_fit<T>(lds, ldq, FitShape{nl, nr, rank, -1}, g.iters, g.fudge, W, wrow, chisq, false);
+            __builtin_amdgcn_wave_barrier();
+            double* wm = g.wm + (static_cast<std::int64_t>(g.slot0 + slot) * nbs + f) * kMaxNl;
+            if (lane < nl) wm[lane] = ok ? wrow[lane] : 0.0;
+        } else {
             const int k = s_fit_row[f], rr = s_fit_rank[f];
-            FitShape sh{k == 0 ? nl : nl - 1, nr, rr, k == 0 ? -1 : nl - k};
+            const FitShape sh{k == 0 ? nl : nl - 1, nr, rr, k == 0 ? -1 : nl - k};
             const int mr = sh.nl * nr;
             if (lane < mr) {
                 const int i = lane / nr, j = lane - (lane / nr) * nr;
-                W.x[lane] = s_xtot[src_of(i, sh.drop) * nr + j];
+                W.x[lane] = sp.xtot[src_of(i, sh.drop) * nr + j];
             }
             __builtin_amdgcn_wave_barrier();
-            double chisq = 0.0;
             const int rf = sh.nl - 1;
-            double* wout = rr == rf ? s_wrf[k] : (k == 0 && rr == rank ? s_wmain : W.sig);
-            const bool ok = als_fit<T>(sQi, ldq, sh, g.iters, g.fudge, W, wout, chisq, true);
+            double* wout = rr == rf ? tb->wrf[k] : (k == 0 && rr == rank ? tb->wmain : W.sig);
+            const bool ok = als_fit<T>(lds, ldq, sh, g.iters, g.fudge, W, wout, chisq, true);
             if (lane == 0) {
-                s_chisq[k][rr] = ok ? chisq : 0.0;
-                s_ok[k][rr] = ok ? 1 : 0;
+                tb->chisq[k][rr] = ok ? chisq : 0.0;
+                tb->ok[k][rr] = ok ? 1 : 0;
             }
         }
-        __syncthreads();
-        const bool main_ok = s_ok[0][rank] != 0;
-        const double* wmain = rank == nl - 1 ? s_wrf[0] : s_wmain;
-        const int dof = dof_of(nl, nr, rank);
-        bool do_se = false;
-        if (main_ok && nbs >= 2) {
-            if (g.jackknife == 2) do_se = true;
-            else if (g.jackknife == 1)
-                do_se = feasible_w(wmain, nl) &&
-                        (!g.se_require_p || chisq_upper(s_chisq[0][rank], dof) >= g.p_se_threshold);
-        }
-        if (do_se) {
-            if (tid == 0) s_next = 0;
-            __syncthreads();
-            for (;;) {
-                int b = 0;
-                if (lane == 0) b = atomicAdd(&s_next, 1);
-                b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-                if (b >= nbs) break;
-                if (lane < m) W.x[lane] = sLOO[static_cast<std::int64_t>(lane) * nbs + b];
-                __builtin_amdgcn_wave_barrier();
-                FitShape sh{nl, nr, rank, -1};
-                double chisq = 0.0;
-                double* wrow = W.sig;  // nl weights; sig is free after the seed
-                const bool ok = als_fit<T>(sQi, ldq, sh, g.iters, g.fudge, W, wrow, chisq, false);
-                __builtin_amdgcn_wave_barrier();
-                if (lane < nl) sWM[static_cast<std::int64_t>(b) * nl + lane] = ok ? wrow[lane] : 0.0;
-            }
-            __syncthreads();
-        }
-
-        // ---- results (wave 0; lane 0 writes the record fields) ----
-        if (tid < 64) {
-            double se = 0.0;
-            if (do_se && lane < nl) se = loo_se(sWM, nbs, nl, lane);
-            write_qpadm_record(out, mi, nl, nr, rank, g.alpha, s_chisq, s_ok, s_wrf, wmain, main_ok, do_se, se,
-                               s_prank);
-        }
-        __syncthreads();
+        __builtin_amdgcn_wave_barrier();
     }
+}
+
+// The result records, a wavefront per model.
+__global__ __launch_bounds__(kQThreads) void qpadm_finish_kernel(QpFitArgs g, int n_models, double alpha,
+                                                                 stp_qpadm_result* __restrict__ results) {
+    __shared__ double s_prob[kQWaves][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int slot = static_cast<int>(blockIdx.x) * kQWaves + wave;
+    if (slot >= n_models) return;
+    const QpLargeModel md = g.models[slot];
+    const QpLargeTables* tb = g.tables + slot;
+    stp_qpadm_result* out = results + md.mi;
+    const int nl = md.nl, nr = md.nr, rank = md.rank;
+    if (!tb->cov_ok) {
+        if (lane == 0) {
+            out->status = 3;  // NonSpdCovariance
+            out->model_index = md.mi;
+            out->nl = 0;
+            out->est_rank = rank;
+            out->dof = dof_of(nl, nr, rank);
+            out->n_rank = 0;
+            out->n_popdrop = 0;
+        }
+        return;
+    }
+    const bool main_ok = tb->ok[0][rank] != 0;
+    const double* wmain = rank == nl - 1 ? tb->wrf[0] : tb->wmain;
+    const bool do_se = qpadm_do_se(main_ok, g.nbs, g.jackknife, wmain, nl, g.se_require_p != 0, tb->chisq[0][rank],
+                                   dof_of(nl, nr, rank), g.p_se_threshold);
+    double se = 0.0;
+    if (do_se) se = loo_se(g.wm + static_cast<std::int64_t>(slot) * g.nbs * kMaxNl, g.nbs, nl);
+    write_qpadm_record(out, md.mi, nl, nr, rank, alpha, tb->chisq, tb->ok, tb->wrf, wmain, main_ok, do_se, se,
+                       s_prob[wave]);
 }
 
 // ---------------------------------------------------------------------------------
@@ -633,52 +644,48 @@ void launch_transpose_survivors(const double* f2, std::int64_t slab, const std::
     STP_LAUNCH_CHECK();
 }
 
-std::size_t qpadm_lds_bytes(int m_max, int ldq, int wave_slice) {
-    const std::size_t a = static_cast<std::size_t>(m_max) * ldq;
-    const std::size_t b = std::max<std::size_t>(a, static_cast<std::size_t>(kQWaves) * wave_slice);
-    return (a + b) * sizeof(double);
+static int host_wave_slice(int nr_max) { return 416 + nr_max * nr_max + (kMaxQpadmNr + 1) / 2 + 1; }
+
+template <class K>
+static void allow_lds(K kernel, std::size_t lds) {
+    if (lds > 64 * 1024)
+        STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
 }
 
-int qpadm_wave_slice(int nr_max) { return 416 + nr_max * nr_max + (kMaxQpadmNr + 1) / 2 + 1; }
+void launch_qpadm_setup(const QpFitArgs& g, int n_models, int m_max, hipStream_t st) {
+    if (n_models <= 0) return;
+    const std::size_t lds = 2 * static_cast<std::size_t>(m_max) * (m_max + 1) * sizeof(double);
+    allow_lds(qpadm_setup_kernel, lds);
+    qpadm_setup_kernel<<<static_cast<unsigned>(n_models), kQThreads, lds, st>>>(g);
+    STP_LAUNCH_CHECK();
+}
 
-void launch_qpadm(int T, const QpadmArgs& args, int n_workgroups, hipStream_t st) {
-    if (args.n_order <= 0) return;
-    const std::size_t lds = qpadm_lds_bytes(args.m_max, args.ldq, args.wave_slice);
-    const dim3 grid(static_cast<unsigned>(n_workgroups));
+void launch_qpadm_fits(int T, const QpFitArgs& g, bool refits, int n_models, int m_max, int nr_max, hipStream_t st) {
+    if (n_models <= 0) return;
+    const int n_parts = refits ? static_cast<int>(ceil_div(g.nbs, kRefitPart)) : 1;
+    const std::size_t lds =
+        (static_cast<std::size_t>(m_max) * (m_max + 1) + static_cast<std::size_t>(kQWaves) * host_wave_slice(nr_max)) *
+        sizeof(double);
     auto go = [&](auto kernel) {
-        if (lds > 64 * 1024)
-            STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        kernel<<<grid, kQThreads, lds, st>>>(args);
+        allow_lds(kernel, lds);
+        kernel<<<static_cast<unsigned>(n_models) * n_parts, kQThreads, lds, st>>>(g, n_parts, refits ? 1 : 0, nr_max);
     };
     switch (T) {
-        case 16: go(qpadm_kernel<16>); break;
-        case 32: go(qpadm_kernel<32>); break;
-        case 48: go(qpadm_kernel<48>); break;
-        case 64: go(qpadm_kernel<64>); break;
+        case 16: go(qpadm_fit_kernel<16>); break;
+        case 32: go(qpadm_fit_kernel<32>); break;
+        case 48: go(qpadm_fit_kernel<48>); break;
+        case 64: go(qpadm_fit_kernel<64>); break;
         default: throw ArgError("qpadm: unsupported system size bucket " + std::to_string(T));
     }
     STP_LAUNCH_CHECK();
 }
 
-int qpadm_threads() { return kQThreads; }
-
-int qpadm_blocks_per_cu(int T, std::size_t lds) {
-    int n = 0;
-    auto q = [&](auto kernel) {
-        if (lds > 64 * 1024)
-            STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        STP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kQThreads, lds));
-    };
-    switch (T) {
-        case 16: q(qpadm_kernel<16>); break;
-        case 32: q(qpadm_kernel<32>); break;
-        case 48: q(qpadm_kernel<48>); break;
-        case 64: q(qpadm_kernel<64>); break;
-        default: throw ArgError("qpadm: unsupported system size bucket " + std::to_string(T));
-    }
-    return n > 0 ? n : 1;
+void launch_qpadm_finish(const QpFitArgs& g, int n_models, double alpha, stp_qpadm_result* out, hipStream_t st) {
+    if (n_models <= 0) return;
+    qpadm_finish_kernel<<<static_cast<unsigned>(ceil_div(n_models, kQWaves)), kQThreads, 0, st>>>(g, n_models, alpha,
+                                                                                                 out);
+    STP_LAUNCH_CHECK();
 }
 
 }  // namespace stp

@@ -10,38 +10,15 @@
 
 namespace stp {
 
-// Model shape limits of the device fit: one f4 entry per lane (m = nl*nr <= 64) and
-// one normal-matrix row per lane (nl*r, r*nr <= 64).
+// Every model runs as four launches over all models of a call: setup (f4 basis, jackknife
+// covariance and its inverse, a workgroup per model), the fit table (rank sweeps of the full
+// model and of each popdrop row), the leave-one-block-out refits, and the record; so one
+// model's refits spread over the whole device, and many models fill it.
+//
+// Model shape limits of the fits with one f4 entry per lane (m = nl*nr <= 64) and one
+// normal-matrix row per lane (nl*r, r*nr <= 64).
 constexpr int kMaxQpadmM = 64;
 constexpr int kMaxQpadmNr = 32;
-
-struct QpadmArgs {
-    const double* f2T;            // survivor-transposed f2: [(i + P*j) * nbs + s]
-    const std::int32_t* bsz;      // survivor block sizes [nbs]
-    int P = 0, nbs = 0;
-    double n_total = 0.0;         // sum of the survivor block sizes
-    // model arena: left[left_off[i] .. left_off[i+1]) are model i's sources,
-    // right[right_off[i] .. right_off[i+1]) its right set (right[0] is the base)
-    const std::int32_t* target;
-    const std::int32_t* left_off;
-    const std::int32_t* left;
-    const std::int32_t* right_off;
-    const std::int32_t* right;
-    const std::int32_t* order;    // models of this launch, in claim order
-    int n_order = 0;
-    unsigned* counter;
-    double fudge = 1e-4;
-    int iters = 20;
-    int rank = -1;
-    double alpha = 0.05;
-    int jackknife = 2;            // 0 none, 1 feasible-only, 2 all
-    int se_require_p = 0;
-    double p_se_threshold = 0.05;
-    double* scratch;              // per workgroup: X/tau [m_max][nbs], LOO [m_max][nbs], wm [nbs][8]
-    std::int64_t scratch_stride = 0;
-    stp_qpadm_result* out;        // indexed by model
-    int m_max = 0, ldq = 0, nr_max = 0, wave_slice = 0;
-};
 
 // ---- models beyond the batched kernel (qpadm_large.hip) -----------------------------
 // Largest f4 basis (sources x (right - 1)), right set and normal system of the large path.
@@ -68,7 +45,6 @@ struct QpLargeTables {
     int ok[STP_QPADM_MAX_NL + 1][STP_QPADM_MAX_NL + 1];
     double wrf[STP_QPADM_MAX_NL + 1][STP_QPADM_MAX_NL];
     double wmain[STP_QPADM_MAX_NL];
-    double prank[STP_QPADM_MAX_NL + 1];
     int cov_ok, pad;
 };
 
@@ -90,7 +66,7 @@ struct QpLargeArgs {
     double* fit = nullptr;         // per-wavefront fit scratch
     std::int64_t fit_stride = 0;
     int m_max = 0, nr_max = 0, t_max = 0;
-    double* wm = nullptr;          // leave-one-block-out weights: slot s, block b at s*nbs*8 + b*nl
+    double* wm = nullptr;          // leave-one-block-out weights: slot s, block b at (s*nbs + b)*8
     stp_qpadm_result* out = nullptr;
     double fudge = 1e-4;
     int iters = 20;
@@ -100,21 +76,68 @@ struct QpLargeArgs {
     double p_se_threshold = 0.05;
 };
 
+// ---- models within the limits above (qpadm.hip, qpadm_rows.hip) -----------------------
+// QpLargeModel and QpLargeTables describe them too; models[0 .. n_models) of a launch share
+// a kernel instance.  slot0 is the index of models[0] among the chunk's models.
+struct QpFitArgs {
+    const double* f2T = nullptr;
+    const std::int32_t* bsz = nullptr;
+    int P = 0, nbs = 0;
+    double n_total = 0.0;
+    const std::int32_t* target = nullptr;
+    const std::int32_t* left = nullptr;
+    const std::int32_t* right = nullptr;
+    const QpLargeModel* models = nullptr;
+    QpLargeTables* tables = nullptr;
+    double* setup = nullptr;       // per-model setup results (qp_setup)
+    double* wm = nullptr;          // leave-one-block-out weights: slot s, block b at (s*nbs + b)*8
+    double fudge = 1e-4;
+    int iters = 20;
+    int jackknife = 2;             // 0 none, 1 feasible-only, 2 all
+    int se_require_p = 0;
+    double p_se_threshold = 0.05;
+    int slot0 = 0;
+};
+
+// A model's setup results: tau and the leave-one-out values [m][nbs], Qinv [m][m], totals.
+struct QpSetup {
+    double *X, *LOO, *Qi, *xtot, *totline;
+};
+__host__ __device__ inline QpSetup qp_setup(double* setup, const QpLargeModel& md, int nbs) {
+    const std::int64_t mn = static_cast<std::int64_t>(md.m) * nbs;
+    QpSetup p;
+    p.X = setup + md.base;
+    p.LOO = p.X + mn;
+    p.Qi = p.LOO + mn;
+    p.xtot = p.Qi + md.m * md.m;
+    p.totline = p.xtot + md.m;
+    return p;
+}
+inline std::size_t qp_setup_doubles(int m, int nbs) {
+    return 2 * static_cast<std::size_t>(m) * nbs + static_cast<std::size_t>(m) * m + 2 * m;
+}
+
+void launch_qpadm_setup(const QpFitArgs& g, int n_models, int m_max, hipStream_t st);
+// The fits of one system-size bucket T by wavefronts with a matrix row per lane: each
+// model's fit table, or (refits) its leave-one-block-out refits.
+void launch_qpadm_fits(int T, const QpFitArgs& g, bool refits, int n_models, int m_max, int nr_max, hipStream_t st);
+// Leave-one-block-out refits with sixteen lanes a fit: whether a model's take that form, the
+// kernel instance, and the launch over models of one instance (g.models, g.tables and g.wm
+// at the chunk's first model plus slot0).
+bool qpadm_rows_fit(int nl, int nr, int rank, int iters);
+int qpadm_rows_class(int nl, int nr);
+void launch_qpadm_rows(const QpFitArgs& g, int cls, int n_models, int m_max, hipStream_t st);
+// The result records, for models of either path.
+void launch_qpadm_finish(const QpFitArgs& g, int n_models, double alpha, stp_qpadm_result* out, hipStream_t st);
+
 std::size_t qpadm_large_setup_doubles(int m, int nbs);
 std::size_t qpadm_large_fit_doubles(int m_max, int nr_max, int t_max);
 int qpadm_large_fit_waves();
 void launch_qpadm_large_setup(const QpLargeArgs& g, hipStream_t st);
 void launch_qpadm_large_fits(const QpLargeArgs& g, int n_workgroups, hipStream_t st);
-void launch_qpadm_large_finish(const QpLargeArgs& g, hipStream_t st);
 
 void launch_survivors(const double* vpair, std::int64_t slab, int n_block, std::int32_t* keep, hipStream_t st);
 void launch_transpose_survivors(const double* f2, std::int64_t slab, const std::int32_t* surv, int nbs, double* f2T,
                                 hipStream_t st);
-std::size_t qpadm_lds_bytes(int m_max, int ldq, int wave_slice);
-int qpadm_wave_slice(int nr_max);
-void launch_qpadm(int T, const QpadmArgs& args, int n_workgroups, hipStream_t st);
-int qpadm_threads();
-// Workgroups of qpadm_kernel<T> that fit on one CU at once with lds bytes of dynamic LDS.
-int qpadm_blocks_per_cu(int T, std::size_t lds);
 
 }  // namespace stp

@@ -20,8 +20,7 @@ namespace stp {
 namespace {
 
 struct ModelShape {
-    int nl, nr, m, T;
-    double cost;
+    int nl, nr;
 };
 
 // The normal-matrix bucket of a model: rank sweeps and LOO fits run at ranks up to
@@ -85,9 +84,7 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
             STP_REQUIRE(right[k] >= 0 && right[k] < P, tag + "right index out of range");
         total_left += nl;
         total_right += nr + 1;
-        const int T = bucket_of(nl, nr, opt.rank);
-        const double t = static_cast<double>(T);
-        shape[i] = ModelShape{nl, nr, nl * nr, T, (nb + 8.0 * nl) * t * t * t};
+        shape[i] = ModelShape{nl, nr};
     }
     STP_REQUIRE(left_off[n_models] == total_left && right_off[n_models] == total_right,
                 "qpadm: offsets are not cumulative");
@@ -113,14 +110,9 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
     STP_REQUIRE(nbs >= 1, "qpadm: no jackknife block survives (every block has partially missing pairs)");
     for (int s : bsz) STP_REQUIRE(s > 0, "qpadm: surviving blocks must have positive sizes");
 
-    // ---- device arena: survivors, sizes, models, per-bucket claim orders ----
-    std::vector<int> order, large;
-    for (int i = 0; i < n_models; ++i) (fits_batched(shape[i].nl, shape[i].nr) ? order : large).push_back(i);
-    const int n_small = static_cast<int>(order.size());
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-        if (shape[a].T != shape[b].T) return shape[a].T < shape[b].T;
-        return shape[a].cost > shape[b].cost;
-    });
+    // ---- device arena: survivors, sizes, models ----
+    std::vector<int> small, large;
+    for (int i = 0; i < n_models; ++i) (fits_batched(shape[i].nl, shape[i].nr) ? small : large).push_back(i);
     std::vector<std::int32_t> arena;
     auto put = [&](const std::int32_t* p, std::size_t n) {
         const std::size_t off = arena.size();
@@ -134,7 +126,6 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
     const std::size_t o_left = put(left, total_left);
     const std::size_t o_roff = put(right_off, n_models + 1);
     const std::size_t o_right = put(right, total_right);
-    const std::size_t o_order = put(order.data(), order.size());
     qp_i32_.ensure(arena.size());
     STP_HIP(hipMemcpyAsync(qp_i32_.get(), arena.data(), arena.size() * sizeof(std::int32_t), hipMemcpyHostToDevice,
                            stream_));
@@ -146,70 +137,36 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
     // ---- launches per bucket ----
     qp_out_.ensure(static_cast<std::size_t>(n_models));
     STP_HIP(hipMemsetAsync(qp_out_.get(), 0, static_cast<std::size_t>(n_models) * sizeof(stp_qpadm_result), stream_));
-    // Each launch group fills every CU to the kernel's occupancy; every workgroup has its
-    // own scratch slice (X, LOO and the LOO weights), sized for the largest group.
-    std::size_t scratch_elems = 0;
-    for (int slot = 0; slot < n_small;) {
-        const int T = shape[order[slot]].T;
-        int end = slot, m_max = 0, nr_max = 0;
-        for (; end < n_small && shape[order[end]].T == T; ++end) {
-            m_max = std::max(m_max, shape[order[end]].m);
-            nr_max = std::max(nr_max, shape[order[end]].nr);
-        }
-        const std::size_t lds = qpadm_lds_bytes(m_max, m_max + 1, qpadm_wave_slice(nr_max));
-        const std::int64_t n_wg = std::min<std::int64_t>(end - slot, qpadm_blocks_per_cu(T, lds) * n_cu_);
-        scratch_elems = std::max(scratch_elems, static_cast<std::size_t>((2 * m_max + STP_QPADM_MAX_NL) * nbs * n_wg));
-        slot = end;
-    }
-    qp_scratch_.ensure(scratch_elems);
-    counter_.ensure(64);
     mark_begin(kQpadm);
-    int slot = 0;
-    int bucket_id = 0;
-    while (slot < n_small) {
-        const int T = shape[order[slot]].T;
-        int end = slot;
-        int m_max = 0, nr_max = 0;
-        while (end < n_small && shape[order[end]].T == T) {
-            m_max = std::max(m_max, shape[order[end]].m);
-            nr_max = std::max(nr_max, shape[order[end]].nr);
-            ++end;
-        }
-        QpadmArgs a{};
+    auto model_of = [&](int mi) {
+        QpLargeModel md{};
+        md.mi = mi;
+        md.l0 = left_off[mi];
+        md.nl = shape[mi].nl;
+        md.r0 = right_off[mi];
+        md.nr = shape[mi].nr;
+        md.m = md.nl * md.nr;
+        md.rank = opt.rank < 0 ? md.nl - 1 : opt.rank;
+        return md;
+    };
+    if (!small.empty()) {
+        QpFitArgs a{};
         a.f2T = qpT_.get();
         a.bsz = qp_i32_.get() + o_bsz;
         a.P = P;
         a.nbs = nbs;
         a.n_total = n_total;
         a.target = qp_i32_.get() + o_tgt;
-        a.left_off = qp_i32_.get() + o_loff;
         a.left = qp_i32_.get() + o_left;
-        a.right_off = qp_i32_.get() + o_roff;
         a.right = qp_i32_.get() + o_right;
-        a.order = qp_i32_.get() + o_order + slot;
-        a.n_order = end - slot;
-        a.counter = counter_.get() + 32 + bucket_id;
         a.fudge = opt.fudge;
         a.iters = opt.als_iterations;
-        a.rank = opt.rank;
-        a.alpha = opt.rank_alpha;
         a.jackknife = opt.jackknife;
         a.se_require_p = opt.se_require_p;
         a.p_se_threshold = opt.p_se_threshold;
-        a.scratch = qp_scratch_.get();
-        a.scratch_stride = static_cast<std::int64_t>(2 * m_max + STP_QPADM_MAX_NL) * nbs;
-        a.out = qp_out_.get();
-        a.m_max = m_max;
-        a.ldq = m_max + 1;
-        a.nr_max = nr_max;
-        a.wave_slice = qpadm_wave_slice(nr_max);
-        const std::size_t lds = qpadm_lds_bytes(a.m_max, a.ldq, a.wave_slice);
-        STP_REQUIRE(lds <= 96 * 1024, "qpadm: model sizes need more LDS than a workgroup has");
-        launch_zero_u32(a.counter, 1, stream_);
-        launch_qpadm(T, a, std::min(qpadm_blocks_per_cu(T, lds) * n_cu_, a.n_order), stream_);
-        slot = end;
-        ++bucket_id;
-        STP_REQUIRE(bucket_id < 32, "qpadm: too many launch groups");
+        std::vector<QpLargeModel> sm;
+        for (int mi : small) sm.push_back(model_of(mi));
+        qpadm_small(a, std::move(sm), opt);
     }
     if (!large.empty()) {
         QpLargeArgs a{};
@@ -229,23 +186,90 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
         a.se_require_p = opt.se_require_p;
         a.p_se_threshold = opt.p_se_threshold;
         std::vector<QpLargeModel> lm;
-        for (int mi : large) {
-            QpLargeModel md{};
-            md.mi = mi;
-            md.l0 = left_off[mi];
-            md.nl = shape[mi].nl;
-            md.r0 = right_off[mi];
-            md.nr = shape[mi].nr;
-            md.m = md.nl * md.nr;
-            md.rank = opt.rank < 0 ? md.nl - 1 : opt.rank;
-            lm.push_back(md);
-        }
+        for (int mi : large) lm.push_back(model_of(mi));
         qpadm_large(a, lm, opt.rank);
     }
     mark_end(kQpadm);
     STP_HIP(hipMemcpyAsync(out, qp_out_.get(), static_cast<std::size_t>(n_models) * sizeof(stp_qpadm_result),
                            hipMemcpyDeviceToHost, stream_));
     sync();
+}
+
+// Models whose fits hold a matrix row per lane: chunks of models whose setup results and
+// refit weights fit a fixed budget; per chunk the models are ordered by kernel instance and
+// each stage is one launch per instance.
+void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, const stp_qpadm_options& opt) {
+    constexpr std::size_t kSetupBudget = std::size_t{1} << 29;   // doubles (4 GiB)
+    constexpr std::size_t kMaxChunk = 16384;                     // models
+    const int nbs = a.nbs;
+    auto cls = [&](const QpLargeModel& md) {
+        return qpadm_rows_fit(md.nl, md.nr, md.rank, a.iters) ? qpadm_rows_class(md.nl, md.nr) : 0;
+    };
+    auto bucket = [&](const QpLargeModel& md) { return bucket_of(md.nl, md.nr, opt.rank); };
+    // largest systems first: the launches that end in a few long fits come first
+    std::stable_sort(models.begin(), models.end(), [&](const QpLargeModel& x, const QpLargeModel& y) {
+        if (bucket(x) != bucket(y)) return bucket(x) > bucket(y);
+        if (cls(x) != cls(y)) return cls(x) > cls(y);
+        return x.m > y.m;
+    });
+    const bool refits = a.jackknife != 0 && nbs >= 2;
+    for (std::size_t i0 = 0; i0 < models.size();) {
+        std::size_t setup = 0, i1 = i0;
+        int m_max = 0;
+        for (; i1 < models.size() && i1 - i0 < kMaxChunk; ++i1) {
+            QpLargeModel& md = models[i1];
+            const std::size_t need = qp_setup_doubles(md.m, nbs) + (refits ? STP_QPADM_MAX_NL * nbs : 0);
+            if (i1 > i0 && setup + need > kSetupBudget) break;
+            md.base = static_cast<std::int64_t>(setup);
+            setup += need;
+            m_max = std::max(m_max, md.m);
+        }
+        const int nm = static_cast<int>(i1 - i0);
+        ql_models_.ensure(nm);
+        ql_tables_.ensure(nm);
+        ql_setup_.ensure(setup);
+        STP_HIP(hipMemcpyAsync(ql_models_.get(), models.data() + i0, nm * sizeof(QpLargeModel), hipMemcpyHostToDevice,
+                               stream_));
+        launch_zero_u32(reinterpret_cast<unsigned*>(ql_tables_.get()),
+                        static_cast<int>(nm * sizeof(QpLargeTables) / sizeof(unsigned)), stream_);
+        a.models = ql_models_.get();
+        a.tables = ql_tables_.get();
+        a.setup = ql_setup_.get();
+        if (refits) {
+            ql_wm_.ensure(static_cast<std::size_t>(nm) * nbs * STP_QPADM_MAX_NL);
+            a.wm = ql_wm_.get();
+        }
+        launch_qpadm_setup(a, nm, m_max, stream_);
+        // runs of models that share a kernel instance
+        auto runs = [&](auto key, auto launch) {
+            for (int s = 0; s < nm;) {
+                int e = s, mm = 0, nn = 0;
+                for (; e < nm && key(models[i0 + e]) == key(models[i0 + s]); ++e) {
+                    mm = std::max(mm, models[i0 + e].m);
+                    nn = std::max(nn, models[i0 + e].nr);
+                }
+                QpFitArgs r = a;
+                r.models += s;
+                r.tables += s;
+                r.slot0 = s;
+                launch(r, models[i0 + s], e - s, mm, nn);
+                s = e;
+            }
+        };
+        runs(bucket, [&](const QpFitArgs& r, const QpLargeModel& md, int n, int mm, int nn) {
+            launch_qpadm_fits(bucket(md), r, false, n, mm, nn, stream_);
+        });
+        if (refits)
+            runs([&](const QpLargeModel& md) { return 128 * bucket(md) + cls(md); },
+                 [&](const QpFitArgs& r, const QpLargeModel& md, int n, int mm, int nn) {
+                     if (cls(md)) launch_qpadm_rows(r, cls(md), n, mm, stream_);
+                     else launch_qpadm_fits(bucket(md), r, true, n, mm, nn, stream_);
+                 });
+        launch_qpadm_finish(a, nm, opt.rank_alpha, qp_out_.get(), stream_);
+        if (i1 < models.size()) sync();   // the next chunk reuses the buffers' host copies
+        i0 = i1;
+    }
+    sync();   // the models (host memory) must outlive their copy
 }
 
 // Models beyond the batched kernel: chunks of models whose setup scratch fits a fixed
@@ -333,7 +357,15 @@ void HipBackend::qpadm_large(QpLargeArgs a, const std::vector<QpLargeModel>& lar
             launch_zero_u32(a.counter, 1, stream_);
             launch_qpadm_large_fits(a, n_wg, stream_);
         }
-        launch_qpadm_large_finish(a, stream_);
+        QpFitArgs f{};
+        f.models = a.models;
+        f.tables = a.tables;
+        f.nbs = nbs;
+        f.wm = a.wm;
+        f.jackknife = a.jackknife;
+        f.se_require_p = a.se_require_p;
+        f.p_se_threshold = a.p_se_threshold;
+        launch_qpadm_finish(f, nm, a.alpha, a.out, stream_);
         // the chunk's task list (host memory) must outlive its copy
         sync();
     }

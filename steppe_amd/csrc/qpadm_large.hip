@@ -518,7 +518,7 @@ __global__ __launch_bounds__(64 * kFitWaves) __attribute__((amdgpu_waves_per_eu(
             const bool ok = als_fit_large(sp.Qi, sp.QT, md.m, Shape{nl, nr, rank, -1}, g.iters, g.fudge, W,
                                           W.wt, chisq, false);
             wsync();
-            double* wm = g.wm + static_cast<std::int64_t>(tk.slot) * g.nbs * kQpMaxNl + static_cast<std::int64_t>(tk.b) * nl;
+            double* wm = g.wm + (static_cast<std::int64_t>(tk.slot) * g.nbs + tk.b) * kQpMaxNl;
             if (lane < nl) wm[lane] = ok ? W.wt[lane] : 0.0;
             continue;
         }
@@ -540,36 +540,6 @@ __global__ __launch_bounds__(64 * kFitWaves) __attribute__((amdgpu_waves_per_eu(
         }
         wsync();
     }
-}
-
-__global__ __launch_bounds__(64 * kFitWaves) void qpl_finish_kernel(QpLargeArgs g) {
-    const int lane = threadIdx.x & 63;
-    const int slot = static_cast<int>(blockIdx.x) * kFitWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (slot >= g.n_models) return;
-    const QpLargeModel md = g.models[slot];
-    QpLargeTables* tb = g.tables + slot;
-    stp_qpadm_result* out = g.out + md.mi;
-    const int nl = md.nl, nr = md.nr, rank = md.rank;
-    if (!tb->cov_ok) {
-        if (lane == 0) {
-            out->status = 3;  // NonSpdCovariance
-            out->model_index = md.mi;
-            out->nl = 0;
-            out->est_rank = rank;
-            out->dof = dof_of(nl, nr, rank);
-            out->n_rank = 0;
-            out->n_popdrop = 0;
-        }
-        return;
-    }
-    const bool main_ok = tb->ok[0][rank] != 0;
-    const double* wmain = rank == nl - 1 ? tb->wrf[0] : tb->wmain;
-    const bool do_se = qpadm_do_se(main_ok, g.nbs, g.jackknife, wmain, nl, g.se_require_p != 0, tb->chisq[0][rank],
-                                   dof_of(nl, nr, rank), g.p_se_threshold);
-    double se = 0.0;
-    if (do_se && lane < nl) se = loo_se(g.wm + static_cast<std::int64_t>(slot) * g.nbs * kQpMaxNl, g.nbs, nl, lane);
-    write_qpadm_record(out, md.mi, nl, nr, rank, g.alpha, tb->chisq, tb->ok, tb->wrf, wmain, main_ok, do_se, se,
-                       tb->prank);
 }
 
 }  // namespace
@@ -597,12 +567,6 @@ void launch_qpadm_large_setup(const QpLargeArgs& g, hipStream_t st) {
 void launch_qpadm_large_fits(const QpLargeArgs& g, int n_workgroups, hipStream_t st) {
     if (g.n_tasks <= 0) return;
     qpl_fit_kernel<<<static_cast<unsigned>(n_workgroups), 64 * kFitWaves, 0, st>>>(g);
-    STP_LAUNCH_CHECK();
-}
-
-void launch_qpadm_large_finish(const QpLargeArgs& g, hipStream_t st) {
-    if (g.n_models <= 0) return;
-    qpl_finish_kernel<<<static_cast<unsigned>(ceil_div(g.n_models, kFitWaves)), 64 * kFitWaves, 0, st>>>(g);
     STP_LAUNCH_CHECK();
 }
 

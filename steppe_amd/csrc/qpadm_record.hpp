@@ -46,21 +46,33 @@ __device__ inline bool qpadm_do_se(bool main_ok, int nbs, int jackknife, const d
     return false;
 }
 
-// Standard error of weight `i` from its leave-one-block-out refits wm[b * nl + i]:
-// the refits are scaled by (nbs - 1) / sqrt(nbs), then the sample standard deviation
-// (mean in plain double, squares summed in double-double).
-__device__ inline double loo_se(const double* wm, int nbs, int nl, int i) {
+// Standard errors of a model's weights from its leave-one-block-out refits
+// wm[b * kQpMaxNl + i], called by one whole wavefront; weight i's lands in lane i.  The
+// refits are scaled by (nbs - 1) / sqrt(nbs), then the sample standard deviation: the mean is
+// a plain double sum in block order (weights that are equal in every refit keep the rounding
+// that gives the reference's standard error), a lane per weight; the squares are summed in
+// double-double across the wavefront.
+__device__ inline double loo_se(const double* wm, int nbs, int nl) {
     using namespace wl;
+    const int lane = lane_id();
     const double scale = static_cast<double>(nbs - 1) / sqrt(static_cast<double>(nbs));
+    const double* own = wm + (lane < nl ? lane : 0);
     double mean = 0.0;
-    for (int b = 0; b < nbs; ++b) mean += wm[static_cast<std::int64_t>(b) * nl + i] * scale;
+#pragma unroll 16
+    for (int b = 0; b < nbs; ++b) mean += own[static_cast<std::int64_t>(b) * kQpMaxNl] * scale;
     mean /= nbs;
-    dd acc{0.0, 0.0};
-    for (int b = 0; b < nbs; ++b) {
-        const double d = wm[static_cast<std::int64_t>(b) * nl + i] * scale - mean;
-        acc = dd_fma(acc, d, d);
+    double se = 0.0;
+    for (int i = 0; i < nl; ++i) {
+        const double mi = rl(mean, i);
+        dd acc{0.0, 0.0};
+        for (int b = lane; b < nbs; b += 64) {
+            const double d = wm[static_cast<std::int64_t>(b) * kQpMaxNl + i] * scale - mi;
+            acc = dd_fma(acc, d, d);
+        }
+        const double s = sqrt(dd_div_d(wave_total_dd(acc), static_cast<double>(nbs - 1)));
+        if (lane == i) se = s;
     }
-    return sqrt(dd_div_d(acc, static_cast<double>(nbs - 1)));
+    return se;
 }
 
 // Fills the record of model `mi` from its fit tables; called by one whole wavefront.
@@ -68,19 +80,43 @@ __device__ inline double loo_se(const double* wm, int nbs, int nl, int i) {
 //   wrf[k][i]:             weights of row k's fit at rank (sources of row k) - 1
 //   wmain[i]:              weights of the full model's fit at `rank`
 //   se:                    lane i < nl: its weight's standard error (when do_se)
-//   prank:                 kQpMaxRanks doubles of scratch (LDS or global)
+//   prob:                  64 doubles of scratch (LDS or global)
 // Lane 0 writes the record fields; lanes < nl write their SE and z.
 __device__ inline void write_qpadm_record(stp_qpadm_result* out, int mi, int nl, int nr, int rank, double alpha,
                                           const double (*chisq)[kQpMaxRanks], const int (*ok)[kQpMaxRanks],
                                           const double (*wrf)[kQpMaxNl], const double* wmain, bool main_ok,
-                                          bool do_se, double se, double* prank) {
+                                          bool do_se, double se, double* prob) {
     using namespace wl;
     const int lane = lane_id();
     const int dof = dof_of(nl, nr, rank);
     const int nrows = nl >= 2 ? nl + 1 : 1;
     const int rmax = min(nl, nr) - 1;
-    // p of each swept rank, one lane per rank
-    if (main_ok && lane <= rmax) prank[lane] = chisq_upper(chisq[0][lane], dof_of(nl, nr, lane));
+    // Every tail probability of the record, one lane each: swept ranks at 0, nested ranks at
+    // 16, popdrop rows at 32, the main fit at 48.
+    {
+        double x = 0.0;
+        int df = 0;
+        if (main_ok) {
+            if (lane <= rmax) {
+                x = chisq[0][lane];
+                df = dof_of(nl, nr, lane);
+            } else if (lane > 16 && lane <= 16 + rmax) {
+                const int rr = lane - 16;
+                x = chisq[0][rr - 1] - chisq[0][rr];
+                df = dof_of(nl, nr, rr - 1) - dof_of(nl, nr, rr);
+            } else if (lane >= 32 && lane < 32 + nrows) {
+                const int nlr = lane == 32 ? nl : nl - 1;
+                if (nlr >= 1) {
+                    x = chisq[lane - 32][nlr - 1];
+                    df = dof_of(nlr, nr, nlr - 1);
+                }
+            } else if (lane == 48) {
+                x = chisq[0][rank];
+                df = dof;
+            }
+            prob[lane] = chisq_upper(x, df);
+        }
+    }
     __builtin_amdgcn_wave_barrier();
     if (lane == 0) {
         stp_qpadm_result* o = out;
@@ -107,13 +143,13 @@ __device__ inline void write_qpadm_record(stp_qpadm_result* out, int mi, int nl,
         } else {
             o->nl = nl;
             o->chisq = chisq[0][rank];
-            o->p = chisq_upper(chisq[0][rank], dof);
+            o->p = prob[48];
             for (int i = 0; i < nl; ++i) o->weight[i] = wmain[i];
             // rank sweep of the full model
             o->n_rank = rmax + 1;
             int f4 = rmax;
             for (int rr = rmax; rr >= 0; --rr)
-                if (prank[rr] > alpha) f4 = rr;
+                if (prob[rr] > alpha) f4 = rr;
             o->f4rank = f4;
             for (int rr = 0; rr <= rmax; ++rr) {
                 o->rank_chisq[rr] = chisq[0][rr];
@@ -124,13 +160,13 @@ __device__ inline void write_qpadm_record(stp_qpadm_result* out, int mi, int nl,
                 o->rankdrop_f4rank[kk] = rr;
                 o->rankdrop_dof[kk] = dof_of(nl, nr, rr);
                 o->rankdrop_chisq[kk] = chisq[0][rr];
-                o->rankdrop_p[kk] = prank[rr];
+                o->rankdrop_p[kk] = prob[rr];
                 if (rr >= 1) {
                     const int ddf = dof_of(nl, nr, rr - 1) - dof_of(nl, nr, rr);
                     const double cd = chisq[0][rr - 1] - chisq[0][rr];
                     o->rankdrop_dofdiff[kk] = ddf;
                     o->rankdrop_chisqdiff[kk] = cd;
-                    o->rankdrop_p_nested[kk] = chisq_upper(cd, ddf);
+                    o->rankdrop_p_nested[kk] = prob[16 + rr];
                 } else {
                     o->rankdrop_dofdiff[kk] = INT_MIN;
                     o->rankdrop_chisqdiff[kk] = __builtin_nan("");
@@ -150,7 +186,7 @@ __device__ inline void write_qpadm_record(stp_qpadm_result* out, int mi, int nl,
                 const int pdof = dof_of(nlr, nr, rf);
                 o->popdrop_dof[k] = pdof;
                 o->popdrop_chisq[k] = rf <= rmx ? chisq[k][rf] : 0.0;
-                o->popdrop_p[k] = rf <= rmx ? chisq_upper(chisq[k][rf], pdof) : 0.0;
+                o->popdrop_p[k] = rf <= rmx ? prob[32 + k] : 0.0;
                 // feasible: every weight of the row's fit in [0, 1] (the dropped
                 // source is NaN and ignored); a failed fit is infeasible
                 bool feas = ok[k][rf] != 0 && nlr > 0;

@@ -30,7 +30,7 @@ __device__ inline int rli(int x, int l) { return __builtin_amdgcn_readlane(x, l)
 // f(std::integral_constant<int, I>) for I = 0 .. N-1, as straight-line code.
 template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
-    [&]<int... I>(std::integer_sequence<int, I...>) {
+    [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
         (f(std::integral_constant<int, I>{}), ...);
     }(std::make_integer_sequence<int, N>{});
 }
@@ -158,6 +158,64 @@ __device__ inline double dd_div_dd(dd a, dd b) {
     const double pe = fma(q, b.hi, -p);
     const double r = (((a.hi - p) - pe) + a.lo) - q * b.lo;
     return q + r / b.hi;
+}
+
+// The value of lane (this lane's DPP source) for a double; every lane active.
+template <int CTRL>
+__device__ inline double dpp(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+// Lane pairings inside a row of 16 lanes that flip lane bits {3..0}, {2..0}, {1, 0}, {0}: the
+// four stages of a sum over the row.
+constexpr int kRowMirror = 0x140, kHalfMirror = 0x141, kQuadMirror = 0x1B, kQuadSwap = 0xB1;
+// Broadcast of lane J of each row of 16 lanes to the row.
+template <int J>
+__device__ inline double row_bcast(double v) {
+    return dpp<0x150 + J>(v);
+}
+// Sum over each row of 16 lanes, the same bits in every lane of the row.
+__device__ inline double row_sum(double v) {
+    v += dpp<kRowMirror>(v);
+    v += dpp<kHalfMirror>(v);
+    v += dpp<kQuadMirror>(v);
+    v += dpp<kQuadSwap>(v);
+    return v;
+}
+template <int CTRL>
+__device__ inline dd dd_dpp_add(dd v) {
+    return dd_add_dd(v, dd{dpp<CTRL>(v.hi), dpp<CTRL>(v.lo)});
+}
+__device__ inline dd dd_xor_add(dd v, int mask) {
+    return dd_add_dd(v, dd{__shfl_xor(v.hi, mask), __shfl_xor(v.lo, mask)});
+}
+// Sum over the wavefront (every lane active), the same bits in every lane.
+__device__ inline dd wave_total_dd(dd v) {
+    v = dd_dpp_add<kRowMirror>(v);
+    v = dd_dpp_add<kHalfMirror>(v);
+    v = dd_dpp_add<kQuadMirror>(v);
+    v = dd_dpp_add<kQuadSwap>(v);
+    const dd r0{rl(v.hi, 0), rl(v.lo, 0)}, r1{rl(v.hi, 16), rl(v.lo, 16)};
+    const dd r2{rl(v.hi, 32), rl(v.lo, 32)}, r3{rl(v.hi, 48), rl(v.lo, 48)};
+    return dd_add_dd(dd_add_dd(r0, r1), dd_add_dd(r2, r3));
+}
+// Four sums over the wavefront (every lane active): lane l holds the sum of v[(l >> 2) & 3].
+// The first two stages add two values at a time, each half of the lanes keeping one.
+__device__ inline dd wave_total4_dd(const dd (&v)[4]) {
+    const int lane = lane_id();
+    const bool b3 = lane & 8, b2 = lane & 4;
+    auto two = [](bool hi, dd a, dd b, auto ctrl) {
+        constexpr int c = decltype(ctrl)::value;
+        const dd keep{hi ? b.hi : a.hi, hi ? b.lo : a.lo}, send{hi ? a.hi : b.hi, hi ? a.lo : b.lo};
+        return dd_add_dd(keep, dd{dpp<c>(send.hi), dpp<c>(send.lo)});
+    };
+    const std::integral_constant<int, kRowMirror> m16{};
+    const std::integral_constant<int, kHalfMirror> m8{};
+    dd r = two(b2, two(b3, v[0], v[2], m16), two(b3, v[1], v[3], m16), m8);
+    r = dd_dpp_add<kQuadMirror>(r);
+    r = dd_dpp_add<kQuadSwap>(r);
+    return dd_xor_add(dd_xor_add(r, 16), 32);
 }
 
 // ---------------------------------------------------------------------------------
