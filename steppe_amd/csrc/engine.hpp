@@ -506,6 +506,7 @@ private:
     DevBuf<stp_qpadm_result> qp_out_;
     // Large-model qpAdm working set (grow-only): model and task lists, fit tables,
     // per-model setup scratch, per-wavefront fit scratch, leave-one-block-out weights.
+    void fetch_hits(std::int64_t n, std::int64_t K, std::vector<SweepHit>& res);
     void qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, const stp_qpadm_options& opt);
     void qpadm_large(QpLargeArgs a, const std::vector<QpLargeModel>& large, int rank_opt);
     DevBuf<QpLargeModel> ql_models_;
@@ -517,7 +518,8 @@ private:
     DevBuf<std::int32_t> fs_i32_, fs_idx_;
     DevBuf<double> fs_out_;
     DevBuf<std::int64_t> fs_i64_;
-    DevBuf<SweepHit> fs_hits_;
+    DevBuf<SweepHit> fs_hits_, fs_select_;
+    DevBuf<unsigned> fs_hist_;
     DevBuf<unsigned long long> fs_count_;
     DevBuf<double> fs_mean_, fs_wroot_;
     DevBuf<GramItem> fs_items_;

@@ -28,6 +28,8 @@
 #include "wave_linalg.hpp"
 
 namespace stp {
+
+void launch_zero_u32(unsigned* p, int n, hipStream_t st);
 namespace {
 
 using namespace wl;
@@ -394,6 +396,71 @@ __device__ inline void wave_append(bool pred, unsigned long long* counter, std::
     ok = pred && static_cast<std::int64_t>(slot_out) < cap;
 }
 
+// ---------------------------------------------------------------------------------
+// The strongest hits of a launch.  A launch can leave millions of hits of which a sweep
+// keeps a thousand: a 120-population f4 sweep (8.2M hits, 262 MB) took 152 ms with all of
+// them copied to the host and selected there, and 3.3 ms with this: they are read twice at
+// HBM speed and about 1.1 K reach the host, which takes the exact K.
+// ---------------------------------------------------------------------------------
+__device__ inline unsigned sweep_bin(double z) {
+    return static_cast<unsigned>(__double_as_longlong(fabs(z)) >> 48);   // sign cleared: < kSweepBins
+}
+
+// Each workgroup counts into its own histogram in LDS (128 KB) and adds what is not zero.
+__global__ __launch_bounds__(1024) void sweep_hist_kernel(SweepSelect a) {
+    extern __shared__ unsigned s_hist[];
+    for (int b = threadIdx.x; b < kSweepBins; b += 1024) s_hist[b] = 0;
+    __syncthreads();
+    const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * 1024;
+    for (std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * 1024 + threadIdx.x; i < a.n; i += step)
+        atomicAdd(&s_hist[sweep_bin(a.hits[i].z)], 1u);
+    __syncthreads();
+    for (int b = threadIdx.x; b < kSweepBins; b += 1024)
+        if (s_hist[b]) atomicAdd(a.hist + b, s_hist[b]);
+}
+
+// One workgroup: thread t owns the bins [32 (1023 - t), +32), so thread order is |z| descending.
+__global__ __launch_bounds__(1024) void sweep_cut_kernel(SweepSelect a) {
+    __shared__ unsigned long long s_sum[1024];
+    constexpr int kOwn = kSweepBins / 1024;
+    const int t = threadIdx.x, b0 = kOwn * (1023 - t);
+    unsigned long long own = 0;
+    for (int b = 0; b < kOwn; ++b) own += a.hist[b0 + b];
+    s_sum[t] = own;
+    if (t == 0) {
+        a.n_out[0] = 0;
+        a.n_out[1] = 0;   // fewer than keep hits: every bin
+    }
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {
+        const unsigned long long v = t >= off ? s_sum[t - off] : 0;
+        __syncthreads();
+        s_sum[t] += v;
+        __syncthreads();
+    }
+    const unsigned long long keep = static_cast<unsigned long long>(a.keep);
+    unsigned long long above = s_sum[t] - own;   // hits in stronger bins
+    if (above < keep && s_sum[t] >= keep)
+        for (int b = kOwn - 1; b >= 0; --b) {
+            above += a.hist[b0 + b];
+            if (above >= keep) {
+                a.n_out[1] = static_cast<unsigned long long>(b0 + b);
+                break;
+            }
+        }
+}
+
+__global__ __launch_bounds__(kThreads) void sweep_compact_kernel(SweepSelect a) {
+    const unsigned cut = static_cast<unsigned>(a.n_out[1]);
+    const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * kThreads;
+    for (std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < a.n; i += step) {
+        unsigned long long slot;
+        bool ok;
+        wave_append(sweep_bin(a.hits[i].z) >= cut, a.n_out, a.n, lane_id(), slot, ok);
+        if (ok) a.out[slot] = a.hits[i];
+    }
+}
+
 __global__ __launch_bounds__(kGramThreads) void f4_gram_kernel(GramArgs a) {
     __shared__ double sE[kGramK * kGramLd];
     __shared__ double sG[2 * kGramRows], sD[2 * kGramRows], sL[2 * kGramRows];
@@ -618,6 +685,19 @@ void launch_f4_gram(const GramArgs& a, hipStream_t st) {
     STP_REQUIRE(a.t.nbs >= 1, "f4 Gram sweep: no surviving block");
     STP_REQUIRE(a.n_items <= 0x7ffffff0LL, "f4 Gram sweep: too many items for one launch");
     f4_gram_kernel<<<dim3(static_cast<unsigned>(round_up(a.n_items, 8))), kGramThreads, 0, st>>>(a);
+    STP_LAUNCH_CHECK();
+}
+
+void launch_sweep_select(const SweepSelect& a, hipStream_t st) {
+    if (a.n <= 0) return;
+    constexpr std::size_t lds = kSweepBins * sizeof(unsigned);
+    STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sweep_hist_kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    launch_zero_u32(a.hist, kSweepBins, st);
+    sweep_hist_kernel<<<static_cast<unsigned>(std::min<std::int64_t>(256, (a.n + 1023) / 1024)), 1024, lds, st>>>(a);
+    sweep_cut_kernel<<<1, 1024, 0, st>>>(a);
+    sweep_compact_kernel<<<static_cast<unsigned>(std::min<std::int64_t>(2048, (a.n + kThreads - 1) / kThreads)), kThreads,
+                           0, st>>>(a);
     STP_LAUNCH_CHECK();
 }
 

@@ -57,6 +57,21 @@ struct SweepArgs {
 };
 void launch_sweep_direct(const SweepArgs& a, hipStream_t st);
 
+// Selection of a launch's strongest hits on the device: hist counts hits by the top 16 bits
+// of |z| (kSweepBins bins in increasing |z|, each about 6% wide), cut finds the highest bin
+// with at least `keep` hits at or above it, compact copies those hits.  The K strongest hits
+// are among them for every K <= keep.
+constexpr int kSweepBins = 1 << 15;
+struct SweepSelect {
+    const SweepHit* hits = nullptr;
+    std::int64_t n = 0;                     // hits in the buffer
+    std::int64_t keep = 0;
+    unsigned* hist = nullptr;               // kSweepBins, zeroed by the launch
+    unsigned long long* n_out = nullptr;    // [0] hits selected, [1] the cut bin
+    SweepHit* out = nullptr;                // room for n hits
+};
+void launch_sweep_select(const SweepSelect& a, hipStream_t st);
+
 // Weighted block means of every f2 series: mean[i + P*j] = sum_s bsz[s] f2T[(i+P*j)*nbs+s] / n.
 void launch_f2_means(const FstatTensor& t, double* mean, hipStream_t st);
 

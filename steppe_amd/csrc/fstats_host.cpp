@@ -204,6 +204,39 @@ void HipBackend::f4ratio(const F2Blocks& h, std::int64_t n, const std::int32_t* 
     std::copy(host.begin() + 2 * n, host.end(), z);
 }
 
+// Appends a launch's hits (fs_hits_[0 .. n)) to res; when the sweep keeps far fewer than
+// there are, only the strongest, selected on the device.
+void HipBackend::fetch_hits(std::int64_t n, std::int64_t K, std::vector<SweepHit>& res) {
+    // Below twice K (or a copy of a megabyte) the selection's three small launches and second
+    // synchronisation cost more than the copy that they save.
+    constexpr std::int64_t kCopyAll = 1 << 15;
+    const SweepHit* from = fs_hits_.get();
+    if (n > std::max(2 * K, kCopyAll)) {
+        fs_select_.ensure(static_cast<std::size_t>(n));
+        fs_hist_.ensure(kSweepBins + 4);
+        SweepSelect a;
+        a.hits = fs_hits_.get();
+        a.n = n;
+        a.keep = K;
+        a.hist = fs_hist_.get();
+        a.n_out = reinterpret_cast<unsigned long long*>(fs_hist_.get() + kSweepBins);
+        a.out = fs_select_.get();
+        launch_sweep_select(a, stream_);
+        unsigned long long got = 0;
+        STP_HIP(hipMemcpyAsync(&got, a.n_out, sizeof(got), hipMemcpyDeviceToHost, stream_));
+        STP_HIP(hipStreamSynchronize(stream_));
+        STP_REQUIRE(got >= static_cast<unsigned long long>(K) && got <= static_cast<unsigned long long>(n),
+                    "fstat_sweep: hit selection out of range");
+        n = static_cast<std::int64_t>(got);
+        from = fs_select_.get();
+    }
+    const std::size_t at = res.size();
+    res.resize(at + static_cast<std::size_t>(n));
+    STP_HIP(hipMemcpyAsync(res.data() + at, from, static_cast<std::size_t>(n) * sizeof(SweepHit),
+                           hipMemcpyDeviceToHost, stream_));
+    STP_HIP(hipStreamSynchronize(stream_));
+}
+
 // The Gram form: items are 128 x 128 row blocks of S for each (c2, c3), grouped into
 // launches of about kGramLaunch statistics (all items of a pair in one launch).
 // Statistics whose variance would be formed with too much cancellation come back as
@@ -250,7 +283,6 @@ void HipBackend::f4_sweep_gram(const FstatTensor& t, const std::vector<std::int3
     fs_hits_.ensure(static_cast<std::size_t>(cap));
     fs_recheck_.ensure(static_cast<std::size_t>(cap));
     fs_count_.ensure(2);
-    std::vector<SweepHit> buf;
     std::size_t i0 = 0;
     for (const auto& [i1, nstat] : cuts) {
         STP_HIP(hipMemsetAsync(fs_count_.get(), 0, 2 * sizeof(unsigned long long), stream_));
@@ -295,11 +327,7 @@ void HipBackend::f4_sweep_gram(const FstatTensor& t, const std::vector<std::int3
             rechecked += static_cast<std::int64_t>(cnt[1]);
         }
         if (cnt[0] > 0) {
-            buf.resize(cnt[0]);
-            STP_HIP(hipMemcpyAsync(buf.data(), fs_hits_.get(), cnt[0] * sizeof(SweepHit), hipMemcpyDeviceToHost,
-                                   stream_));
-            STP_HIP(hipStreamSynchronize(stream_));
-            res.insert(res.end(), buf.begin(), buf.end());
+            fetch_hits(static_cast<std::int64_t>(cnt[0]), K, res);
             keep_top(res, K, filter, tau);
         }
         i0 = i1;
@@ -371,7 +399,6 @@ void HipBackend::fstat_sweep(const F2Blocks& h, const FstatSweepRequest& req, Fs
         a.hits = fs_hits_.get();
         a.n_hits = fs_count_.get();
         a.cap = chunk;
-        std::vector<SweepHit> buf;
         for (std::int64_t r0 = 0; r0 < static_cast<std::int64_t>(total); r0 += chunk) {
             a.r0 = r0;
             a.count = std::min<std::int64_t>(chunk, static_cast<std::int64_t>(total) - r0);
@@ -383,11 +410,7 @@ void HipBackend::fstat_sweep(const F2Blocks& h, const FstatSweepRequest& req, Fs
             STP_HIP(hipStreamSynchronize(stream_));
             STP_REQUIRE(nh <= static_cast<unsigned long long>(a.count), "fstat_sweep: hit count exceeds the launch");
             if (nh == 0) continue;
-            buf.resize(nh);
-            STP_HIP(hipMemcpyAsync(buf.data(), fs_hits_.get(), nh * sizeof(SweepHit), hipMemcpyDeviceToHost,
-                                   stream_));
-            STP_HIP(hipStreamSynchronize(stream_));
-            res.insert(res.end(), buf.begin(), buf.end());
+            fetch_hits(static_cast<std::int64_t>(nh), K, res);
             keep_top(res, K, req.filter, tau);
         }
     }
