@@ -15,6 +15,8 @@
 // lockstep so that each round's unscored neighbours are fitted in one fleet.
 #include <chrono>
 #include <cmath>
+#include <functional>
+#include <future>
 #include <limits>
 #include <memory>
 #include <unordered_map>
@@ -221,10 +223,16 @@ QgSearchResult HipBackend::qpgraph_search(const F2Blocks& f2, const std::vector<
             std::vector<std::vector<qgenum::Candidate>> nb(K);
             want.clear();
             bool any = false;
+            // the seeds' moves in parallel (a future hands an exception on to this thread)
+            std::vector<std::future<std::vector<qgenum::Candidate>>> moves(K);
+            for (int k = 0; k < K; ++k)
+                if (active[k])
+                    moves[k] = std::async(std::launch::async, qgenum::neighbors, std::cref(cur[k]), std::cref(pops),
+                                          max_nadmix);
             for (int k = 0; k < K; ++k) {
                 if (!active[k]) continue;
                 any = true;
-                nb[k] = qgenum::neighbors(cur[k], pops, max_nadmix);
+                nb[k] = moves[k].get();
                 for (const auto& c : nb[k]) want.push_back(&c);
             }
             if (!any) break;
