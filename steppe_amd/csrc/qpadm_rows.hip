@@ -1,19 +1,19 @@
-// steppe_amd/csrc/qpadm_rows.hip — leave-one-block-out qpAdm refits, one fit per row of 16
-// lanes (four fits per wavefront).
+// steppe_amd/csrc/qpadm_rows.hip — leave-one-block-out qpAdm refits, one fit per group of 16
+// or 8 lanes (four or eight fits per wavefront).
 //
 // A model with jackknife standard errors is refitted nb (hundreds of) times on the same
 // Qinv: nearly all of a qpAdm call.  A fit is a chain of small systems (t = nl r and r nr
 // unknowns); a wavefront that works on one fit with a matrix row per lane keeps t of its 64
 // lanes and spends two lane reads per element of every elimination step.  Here lane j of a
-// 16-lane row owns column j of the f4 matrix (right population j + 1) of one fit:
+// 16- or 8-lane group owns column j of the f4 matrix (right population j + 1) of one fit:
 //
 //   B-step  lane j holds the r rows (p, j) of the normal matrix in registers, so an element of
-//           Qinv read from LDS serves every p, A is the same in all 16 lanes, and the matrix
-//           is built without any exchange.
+//           Qinv read from LDS serves every p, A is the same in all its lanes, and the
+//           matrix is built without any exchange.
 //   A-step  lane j forms W[(i, j), (i', p')] = sum_j' Qinv[(i, j), (i', j')] B[p', j'] and
 //           leaves it in LDS; lane a then sums its rows of the normal matrix over j.
-//   LU      the pivot (the largest entry, ties to the first row) by a 4-stage reduction over
-//           the row of lanes; its owner writes the pivot row to LDS and every lane reads it.
+//   LU      the pivot (the largest entry, ties to the first row) by a 4- or 3-stage reduction
+//           over the group; its owner writes the pivot row to LDS and every lane reads it.
 //   Seed    one-sided Jacobi on the columns: the rotations of the (p, q) loops that share
 //           p + q touch different columns and run at once, lane j with lane p + q - j.
 //
@@ -26,8 +26,11 @@
 // Bound by VALU issue (the eliminations' multiply-subtracts, a third of them on lanes past
 // nr) and, for the small systems, by the pivot reductions.  On MI355X with 744 blocks: 1000
 // models of 2-5 sources and 6-12 right populations 1,061 ms as a workgroup per model and a
-// wavefront per fit, 204 ms so (refits and everything before them); a rotation of 1330
-// models of 2-3 sources 242 -> 51 ms; one model of 2 sources 43.5 -> 0.58 ms.
+// wavefront per fit, 165 ms so (the whole call; 204 ms with 16 lanes for every fit, which
+// leaves half of them idle up to 8 columns); a rotation of 1330 models of 2-3 sources against
+// 8 right populations 242 -> 31 ms (51); one model of 2 sources 43.5 -> 0.58 ms.  Columns
+// padded to 6, 8, 10, 12 with straight-line sums instead of a test per column: the same time
+// at 3 sources, 2.3 times slower at 5 (spills).
 
 #include <climits>
 #include <cmath>
@@ -48,16 +51,19 @@ using namespace wl;
 #define STP_INLINE __attribute__((always_inline))
 
 constexpr int kWaves = 4;
-constexpr int kFits = 4 * kWaves;   // fits of a workgroup
 
 __device__ inline double lane_perm(int byte_index, double v) {
     return __hiloint2double(__builtin_amdgcn_ds_bpermute(byte_index, __double2hiint(v)),
                             __builtin_amdgcn_ds_bpermute(byte_index, __double2loint(v)));
 }
 
+// Lanes a fit: eight where they hold its columns.
+constexpr int lanes_of(int nr) { return nr <= 8 ? 8 : 16; }
+
 template <int NL, int NR>
 struct RowShape {
-    static constexpr int R = NL - 1, TA = NL * R, RA = (TA + 15) / 16;
+    static constexpr int G = lanes_of(NR), kFits = kWaves * 64 / G;   // lanes a fit, fits of a workgroup
+    static constexpr int R = NL - 1, TA = NL * R, RA = (TA + G - 1) / G;
     // LDS doubles of a fit: W of one i' [R][m], y [m], B [R][NR], a pivot row with its
     // right-hand side
     static constexpr int kRow = (TA > NR * R ? TA : NR * R) + 2;
@@ -74,13 +80,13 @@ __device__ inline void best_stage(long long& key, int& pos) {
     pos = take ? p2 : pos;
 }
 
-// LU solve with partial pivoting of one system per row of 16 lanes, as lu_solve_rows: each
+// LU solve with partial pivoting of one system per group of G lanes, as lu_solve_rows: each
 // lane holds ROWS matrix rows (M, right-hand side b, logical position pos; -1 for a row that
 // is none).  Storage column c is unknown order(c) when it is one of the system's (order
 // ascending with c, the same in all lanes; negative otherwise).  buf: COLS + 2 doubles of the
 // fit's LDS, 16-byte aligned.  found(c, x) receives each unknown in every lane; false for an
 // exactly zero pivot.
-template <int ROWS, int COLS, class Order, class Found>
+template <int G, int ROWS, int COLS, class Order, class Found>
 __device__ __forceinline__ bool row_solve(double (&M)[ROWS][COLS], double (&b)[ROWS], int (&pos)[ROWS], double* buf,
                                           Order&& order, Found&& found) {
     bool ok = true;
@@ -97,7 +103,7 @@ __device__ __forceinline__ bool row_solve(double (&M)[ROWS][COLS], double (&b)[R
                 key = take ? mine : key;
                 at = take ? pos[p] : at;
             }
-            best_stage<kRowMirror>(key, at);
+            if constexpr (G == 16) best_stage<kRowMirror>(key, at);
             best_stage<kHalfMirror>(key, at);
             best_stage<kQuadMirror>(key, at);
             best_stage<kQuadSwap>(key, at);
@@ -165,15 +171,16 @@ __device__ __forceinline__ bool row_solve(double (&M)[ROWS][COLS], double (&b)[R
     return ok;
 }
 
-// One fit in each row of 16 lanes: x[i] is the f4 entry (i, lane), Q the model's Qinv in LDS
+// One fit in each group of lanes: x[i] is the f4 entry (i, lane), Q the model's Qinv in LDS
 // (leading dimension ldq), sl the fit's slice of LDS.  Lanes past nr run on row 0's values,
-// hold no matrix row and are never read.  Returns ok; w is the same in the 16 lanes.
+// hold no matrix row and are never read.  Returns ok; w is the same in the
+// group's lanes.
 template <int NL, int NR>
 __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int iters, double fudge,
                                         const double (&x)[NL], double* sl, double (&w)[NL]) {
     using S = RowShape<NL, NR>;
-    constexpr int R = S::R, TA = S::TA, RA = S::RA;
-    const int j = lane_id() & 15;
+    constexpr int G = S::G, R = S::R, TA = S::TA, RA = S::RA;
+    const int j = lane_id() & (G - 1);
     const bool act = j < nr;
     const int ja = act ? j : 0;
     const double* Qj = Q + ja * ldq;   // row (0, j); row (i, j) is i * nr * ldq further
@@ -189,7 +196,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
         static_for<NR>([&](auto jc) STP_INLINE {
             constexpr int jj = decltype(jc)::value;
             if (jj < nr) {
-                const double xv = row_bcast<jj>(x[ii]);
+                const double xv = group_bcast<G, jj>(x[ii]);
                 const double* q = Q + ii * qi + jj * ldq + ja;
 #pragma unroll
                 for (int i = 0; i < NL; ++i) y[i] += q[i * nr] * xv;
@@ -208,7 +215,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
 #pragma unroll
         for (int e = 0; e < NR; ++e) V[e] = e == j ? 1.0 : 0.0;
         bool done = false;
-        const int lane0 = lane_id() & ~15;
+        const int lane0 = lane_id() & ~(G - 1);
         for (int sweep = 0; sweep < 60 && __ballot(!done); ++sweep) {
             double off = 0.0;
             for (int s = 1; s <= 2 * nr - 3; ++s) {
@@ -243,7 +250,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
                         V[e] = rot ? v : V[e];
                     }
             }
-            done = done || row_sum(off) < 1e-30;
+            done = done || group_sum<G>(off) < 1e-30;
         }
         double ss = 0.0;
 #pragma unroll
@@ -254,7 +261,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
         int so[NR];
         static_for<NR>([&](auto ec) STP_INLINE {
             constexpr int e = decltype(ec)::value;
-            sv[e] = row_bcast<e>(sig);
+            sv[e] = group_bcast<G, e>(sig);
             so[e] = e;
         });
 #pragma unroll
@@ -284,13 +291,13 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
 
     double A[NL][R];
     for (int it = 0; it < iters; ++it) {
-        // ---- A-step: unknowns A[i][p] at i R + p, lane a holding rows a and 16 + a ----
+        // ---- A-step: unknowns A[i][p] at i R + p, lane a holding rows a, G + a, ... ----
         {
             double bb[R][NR];
             static_for<NR>([&](auto jc) STP_INLINE {
                 constexpr int jj = decltype(jc)::value;
 #pragma unroll
-                for (int p = 0; p < R; ++p) bb[p][jj] = row_bcast<jj>(B[p]);
+                for (int p = 0; p < R; ++p) bb[p][jj] = group_bcast<G, jj>(B[p]);
             });
             if (act)
 #pragma unroll
@@ -300,7 +307,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
             int pos[RA], ro[RA];
 #pragma unroll
             for (int q = 0; q < RA; ++q) {
-                const int a = j + 16 * q, ac = min(a, TA - 1), ia = ac / R, pa = ac - ia * R;
+                const int a = j + G * q, ac = min(a, TA - 1), ia = ac / R, pa = ac - ia * R;
                 pos[q] = a < TA ? a : -1;
                 ro[q] = ia * nr;
                 b[q] = 0.0;
@@ -346,15 +353,15 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
             double tr = 0.0;
             static_for<TA>([&](auto cc) STP_INLINE {
                 constexpr int c = decltype(cc)::value;
-                tr += row_bcast<c % 16>(dg[c / 16]);
+                tr += group_bcast<G, c % G>(dg[c / G]);
             });
             const double ft = fudge * tr;
             static_for<TA>([&](auto cc) STP_INLINE {
                 constexpr int c = decltype(cc)::value;
-                const double v = M[c / 16][c] + ft;
-                M[c / 16][c] = j == c % 16 ? v : M[c / 16][c];
+                const double v = M[c / G][c] + ft;
+                M[c / G][c] = j == c % G ? v : M[c / G][c];
             });
-            const bool ok = row_solve<RA, TA>(
+            const bool ok = row_solve<G, RA, TA>(
                 M, b, pos, sl, [](auto cc) STP_INLINE { return decltype(cc)::value; },
                 [&](auto cc, double v) STP_INLINE {
                     constexpr int c = decltype(cc)::value;
@@ -412,7 +419,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
             for (int p = 0; p < R; ++p)
                 static_for<NR>([&](auto jc) STP_INLINE {
                     constexpr int jj = decltype(jc)::value;
-                    if (jj < nr) tr += row_bcast<jj>(dg[p]);
+                    if (jj < nr) tr += group_bcast<G, jj>(dg[p]);
                 });
             const double ft = fudge * tr;
             static_for<NR>([&](auto jc) STP_INLINE {
@@ -423,7 +430,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
                     M[p][p * NR + jj] = j == jj ? v : M[p][p * NR + jj];
                 }
             });
-            const bool ok = row_solve<R, R * NR>(
+            const bool ok = row_solve<G, R, R * NR>(
                 M, b, pos, sl,
                 [&](auto cc) STP_INLINE {
                     constexpr int c = decltype(cc)::value;
@@ -455,7 +462,7 @@ __device__ __forceinline__ bool row_fit(const double* Q, int ldq, int nr, int it
         s += 1.0 * 1.0;
         M[0][c] = s;
     }
-    const bool ok = row_solve<1, NL>(
+    const bool ok = row_solve<G, 1, NL>(
         M, b, pos, sl, [](auto cc) STP_INLINE { return decltype(cc)::value; },
         [&](auto cc, double v) STP_INLINE { w[decltype(cc)::value] = v; });
     double sum = 0.0;
@@ -497,15 +504,16 @@ void qpadm_rows_kernel(QpFitArgs g, int n_parts) {
         lds[a * ldq + (e - a * m)] = sp.Qi[e];
     }
     __syncthreads();
-    const int fit = tid >> 4, j = tid & 15;
-    const int b = part * kFits + fit;
+    using S = RowShape<NL, NR>;
+    const int fit = tid / S::G, j = tid & (S::G - 1);
+    const int b = part * S::kFits + fit;
     if (__ballot(b < nbs) == 0) return;          // a wavefront past the last block
     double x[NL], w[NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i)
         x[i] = sp.LOO[static_cast<std::int64_t>(i * nr + min(j, nr - 1)) * nbs + min(b, nbs - 1)];
     const int q_lds = (m * ldq + 1) & ~1;
-    row_fit<NL, NR>(lds, ldq, nr, g.iters, g.fudge, x, lds + q_lds + fit * RowShape<NL, NR>::slice(m), w);
+    row_fit<NL, NR>(lds, ldq, nr, g.iters, g.fudge, x, lds + q_lds + fit * S::slice(m), w);
     if (b >= nbs) return;
     double* wm = g.wm + (static_cast<std::int64_t>(g.slot0 + slot) * nbs + b) * STP_QPADM_MAX_NL;
 #pragma unroll
@@ -523,31 +531,35 @@ bool qpadm_rows_fit(int nl, int nr, int rank, int iters) {
 
 int qpadm_rows_class(int nl, int nr) { return 8 * nl + (nr <= 8 ? 0 : nr <= 12 ? 1 : 2); }
 
+template <int NL, int NR>
+static void launch_rows(const QpFitArgs& g, int n_models, int m_max, hipStream_t st) {
+    using S = RowShape<NL, NR>;
+    const int n_parts = static_cast<int>(ceil_div(g.nbs, S::kFits));
+    const std::size_t lds =
+        (static_cast<std::size_t>((m_max * (m_max | 1) + 1) & ~1) + S::kFits * S::slice(m_max)) * sizeof(double);
+    if (lds > 64 * 1024)
+        STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(qpadm_rows_kernel<NL, NR>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    qpadm_rows_kernel<NL, NR><<<static_cast<unsigned>(n_models * n_parts), 64 * kWaves, lds, st>>>(g, n_parts);
+    STP_LAUNCH_CHECK();
+}
+
 void launch_qpadm_rows(const QpFitArgs& g, int cls, int n_models, int m_max, hipStream_t st) {
-    const int n_parts = static_cast<int>(ceil_div(g.nbs, kFits));
     if (n_models <= 0) return;
-    auto go = [&](auto kernel, int slice) {
-        const std::size_t lds = (static_cast<std::size_t>((m_max * (m_max | 1) + 1) & ~1) + kFits * slice) * sizeof(double);
-        if (lds > 64 * 1024)
-            STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        kernel<<<static_cast<unsigned>(n_models * n_parts), 64 * kWaves, lds, st>>>(g, n_parts);
-    };
     switch (cls) {
-        case 8 * 2: go(qpadm_rows_kernel<2, 8>, RowShape<2, 8>::slice(m_max)); break;
-        case 8 * 2 + 1: go(qpadm_rows_kernel<2, 12>, RowShape<2, 12>::slice(m_max)); break;
-        case 8 * 2 + 2: go(qpadm_rows_kernel<2, 16>, RowShape<2, 16>::slice(m_max)); break;
-        case 8 * 3: go(qpadm_rows_kernel<3, 8>, RowShape<3, 8>::slice(m_max)); break;
-        case 8 * 3 + 1: go(qpadm_rows_kernel<3, 12>, RowShape<3, 12>::slice(m_max)); break;
-        case 8 * 3 + 2: go(qpadm_rows_kernel<3, 16>, RowShape<3, 16>::slice(m_max)); break;
-        case 8 * 4: go(qpadm_rows_kernel<4, 8>, RowShape<4, 8>::slice(m_max)); break;
-        case 8 * 4 + 1: go(qpadm_rows_kernel<4, 12>, RowShape<4, 12>::slice(m_max)); break;
-        case 8 * 4 + 2: go(qpadm_rows_kernel<4, 16>, RowShape<4, 16>::slice(m_max)); break;
-        case 8 * 5: go(qpadm_rows_kernel<5, 8>, RowShape<5, 8>::slice(m_max)); break;
-        case 8 * 5 + 1: go(qpadm_rows_kernel<5, 12>, RowShape<5, 12>::slice(m_max)); break;
+        case 8 * 2: return launch_rows<2, 8>(g, n_models, m_max, st);
+        case 8 * 2 + 1: return launch_rows<2, 12>(g, n_models, m_max, st);
+        case 8 * 2 + 2: return launch_rows<2, 16>(g, n_models, m_max, st);
+        case 8 * 3: return launch_rows<3, 8>(g, n_models, m_max, st);
+        case 8 * 3 + 1: return launch_rows<3, 12>(g, n_models, m_max, st);
+        case 8 * 3 + 2: return launch_rows<3, 16>(g, n_models, m_max, st);
+        case 8 * 4: return launch_rows<4, 8>(g, n_models, m_max, st);
+        case 8 * 4 + 1: return launch_rows<4, 12>(g, n_models, m_max, st);
+        case 8 * 4 + 2: return launch_rows<4, 16>(g, n_models, m_max, st);
+        case 8 * 5: return launch_rows<5, 8>(g, n_models, m_max, st);
+        case 8 * 5 + 1: return launch_rows<5, 12>(g, n_models, m_max, st);
         default: throw ArgError("qpadm: unsupported row-fit class " + std::to_string(cls));
     }
-    STP_LAUNCH_CHECK();
 }
 
 }  // namespace stp

@@ -175,9 +175,23 @@ template <int J>
 __device__ inline double row_bcast(double v) {
     return dpp<0x150 + J>(v);
 }
-// Sum over each row of 16 lanes, the same bits in every lane of the row.
-__device__ inline double row_sum(double v) {
-    v += dpp<kRowMirror>(v);
+// Broadcast of lane J of each group of G = 16 or 8 lanes to the group.
+template <int G, int J>
+__device__ inline double group_bcast(double v) {
+    if constexpr (G == 16) {
+        return row_bcast<J>(v);
+    } else {
+        // the row's second half (banks 2 and 3) takes its own lane
+        const double lower = row_bcast<J>(v);
+        const int lo = __builtin_amdgcn_update_dpp(__double2loint(lower), __double2loint(v), 0x158 + J, 0xF, 0xC, false);
+        const int hi = __builtin_amdgcn_update_dpp(__double2hiint(lower), __double2hiint(v), 0x158 + J, 0xF, 0xC, false);
+        return __hiloint2double(hi, lo);
+    }
+}
+// Sum over each group of G = 16 or 8 lanes, the same bits in every lane of the group.
+template <int G>
+__device__ inline double group_sum(double v) {
+    if constexpr (G == 16) v += dpp<kRowMirror>(v);
     v += dpp<kHalfMirror>(v);
     v += dpp<kQuadMirror>(v);
     v += dpp<kQuadSwap>(v);
