@@ -20,8 +20,8 @@
 // The derivative is that of the active-set branch; at a change of active set the
 // score has a kink and this is one of its one-sided derivatives.
 //
-// One workgroup of 256 threads evaluates one instance (a topology, its data and a
-// theta), persistent over the instances of the launch.  Everything per instance sits in
+// One workgroup of 256 threads, or of one wavefront (qg_shape), evaluates one instance (a
+// topology, its data and a theta), persistent over the instances of the launch.  Everything per instance sits in
 // LDS; Qinv is read from global memory (row-major).  The NNLS and the small LU solves
 // run on wavefront 0 with one matrix row per lane.
 
@@ -213,7 +213,7 @@ struct EvalShared {
 // and in the joint mode d score / d bl to L.blbar.  fit (global, may be null) receives
 // P bl.  Returns false on every thread when an edge-length system is singular; the
 // score is then +inf.
-template <int T>
+template <int T, int NT>
 __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const double* __restrict__ G,
                             const double* __restrict__ f, int mode, const EvalLds& L, const EvalShared& sh,
                             double* fit, bool warm = false) {
@@ -223,7 +223,7 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
     const std::int32_t* ia = g.iarena;
     const int np = tp.npair, ne = tp.ne, npop = tp.npop, ncc = npop - 1, D = tp.nadmix, npath = tp.npath;
     // ---- leaf weights from the path tables ----
-    for (int p = tid; p < npath; p += kThreads) {
+    for (int p = tid; p < npath; p += NT) {
         double w = 1.0;
         for (int t = ia[tp.o_pae_off + p]; t < ia[tp.o_pae_off + p + 1]; ++t) {
             const int id = ia[tp.o_pae_id + t];
@@ -232,28 +232,28 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
         }
         L.path[p] = w;
     }
-    for (int x = tid; x < ne * npop; x += kThreads) L.pw[x] = g.darena[tp.o_pwts0 + x];
+    for (int x = tid; x < ne * npop; x += NT) L.pw[x] = g.darena[tp.o_pwts0 + x];
     __syncthreads();
-    for (int gr = tid; gr < tp.ngrp; gr += kThreads) {
+    for (int gr = tid; gr < tp.ngrp; gr += NT) {
         double s = 0.0;
         for (int t = ia[tp.o_grp_off + gr]; t < ia[tp.o_grp_off + gr + 1]; ++t) s += L.path[ia[tp.o_grp_paths + t]];
         L.pw[ia[tp.o_grp_edge + gr] + ne * ia[tp.o_grp_leaf + gr]] = s;
     }
     __syncthreads();
-    for (int x = tid; x < ne * ncc; x += kThreads) {
+    for (int x = tid; x < ne * ncc; x += NT) {
         const int col = x / ne, e = x - (x / ne) * ne;
         const int leaf = col < tp.base ? col : col + 1;
         L.pc[x] = L.pw[e + ne * leaf] - L.pw[e + ne * tp.base];
     }
     __syncthreads();
-    for (int x = tid; x < np * ne; x += kThreads) {
+    for (int x = tid; x < np * ne; x += NT) {
         const int k = x / ne, e = x - (x / ne) * ne;
         L.P[x] = L.pc[e + ne * ia[tp.o_cmb1 + k]] * L.pc[e + ne * ia[tp.o_cmb2 + k]];
     }
     __syncthreads();
     if (mode != 2) {
         // ---- W = G P, qf = G f ----
-        for (int x = tid; x < np * ne; x += kThreads) {
+        for (int x = tid; x < np * ne; x += NT) {
             const int r = x / ne, e = x - (x / ne) * ne;
             const double* Gr = G + static_cast<std::int64_t>(r) * np;
             double acc = 0.0;
@@ -261,7 +261,7 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
             for (int c = 0; c < np; ++c) acc += Gr[c] * L.P[c * ne + e];
             L.W[x] = acc;
         }
-        for (int r = tid; r < np; r += kThreads) {
+        for (int r = tid; r < np; r += NT) {
             const double* Gr = G + static_cast<std::int64_t>(r) * np;
             double acc = 0.0;
 #pragma unroll 8
@@ -270,13 +270,13 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
         }
         __syncthreads();
         // ---- cc = P^T W, q = P^T qf ----
-        for (int x = tid; x < ne * ne; x += kThreads) {
+        for (int x = tid; x < ne * ne; x += NT) {
             const int e1 = x / ne, e2 = x - (x / ne) * ne;
             double acc = 0.0;
             for (int r = 0; r < np; ++r) acc += L.P[r * ne + e1] * L.W[r * ne + e2];
             L.C[x] = acc;
         }
-        for (int e1 = tid; e1 < ne; e1 += kThreads) {
+        for (int e1 = tid; e1 < ne; e1 += NT) {
             double rr = 0.0;
             for (int r = 0; r < np; ++r) rr += L.P[r * ne + e1] * L.qf[r];
             L.q[e1] = rr;
@@ -290,7 +290,7 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
             *sh.ok = 1;
         }
         __syncthreads();
-        for (int e = tid; e < ne; e += kThreads) {
+        for (int e = tid; e < ne; e += NT) {
             L.sc[e] = sqrt(L.C[e * ne + e]);
             L.q1[e] = L.q[e] / L.sc[e];
         }
@@ -317,18 +317,18 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
             __syncthreads();
             return false;
         }
-        for (int e = tid; e < ne; e += kThreads) L.bl[e] = L.lam[e] / L.sc[e];
+        for (int e = tid; e < ne; e += NT) L.bl[e] = L.lam[e] / L.sc[e];
     }
     __syncthreads();
     // ---- residual and score ----
-    for (int k = tid; k < np; k += kThreads) {
+    for (int k = tid; k < np; k += NT) {
         double fv = 0.0;
         for (int e = 0; e < ne; ++e) fv += L.P[k * ne + e] * L.bl[e];
         L.res[k] = f[k] - fv;
         if (fit) fit[k] = fv;
     }
     __syncthreads();
-    for (int a = tid; a < np; a += kThreads) {
+    for (int a = tid; a < np; a += NT) {
         const double* Ga = G + static_cast<std::int64_t>(a) * np;
         double row = 0.0, col = 0.0;
 #pragma unroll 8
@@ -351,16 +351,16 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
         return true;
     }
     // ---- adjoint ----
-    for (int k = tid; k < np; k += kThreads) L.u[k] = L.Gr[k] + L.GTr[k];  // rbar
+    for (int k = tid; k < np; k += NT) L.u[k] = L.Gr[k] + L.GTr[k];  // rbar
     __syncthreads();
-    for (int e = tid; e < ne; e += kThreads) {
+    for (int e = tid; e < ne; e += NT) {
         double s = 0.0;
         for (int k = 0; k < np; ++k) s += L.P[k * ne + e] * L.u[k];
         L.blbar[e] = -s;
     }
     __syncthreads();
     if (mode == 2) {
-        for (int x = tid; x < np * ne; x += kThreads) {
+        for (int x = tid; x < np * ne; x += NT) {
             const int k = x / ne, e = x - (x / ne) * ne;
             L.W[x] = -L.u[k] * L.bl[e];
         }
@@ -388,20 +388,20 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
         }
         __syncthreads();
         const double kappa = sh.scal[0];
-        for (int c = tid; c < np; c += kThreads) {
+        for (int c = tid; c < np; c += NT) {
             double s = 0.0;
             for (int e = 0; e < ne; ++e) s += L.P[c * ne + e] * L.lam[e];
             L.v[c] = s;  // P lambda
         }
         __syncthreads();
-        for (int k = tid; k < np; k += kThreads) {
+        for (int k = tid; k < np; k += NT) {
             double s = 0.0;
 #pragma unroll 8
             for (int c = 0; c < np; ++c) s += G[static_cast<std::int64_t>(c) * np + k] * L.v[c];
             L.qf[k] = s;  // G^T P lambda
         }
         __syncthreads();
-        for (int x = tid; x < np * ne; x += kThreads) {
+        for (int x = tid; x < np * ne; x += NT) {
             const int k = x / ne, e = x - (x / ne) * ne;
             double w2 = 0.0;
 #pragma unroll 8
@@ -411,7 +411,7 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
     }
     __syncthreads();
     // ---- Pbar -> pcbar -> pwbar -> pathbar -> thetabar ----
-    for (int e = tid; e < ne; e += kThreads) {
+    for (int e = tid; e < ne; e += NT) {
         for (int c = 0; c < ncc; ++c) L.pcbar[e + ne * c] = 0.0;
         for (int k = 0; k < np; ++k) {
             const int a = ia[tp.o_cmb1 + k], b = ia[tp.o_cmb2 + k];
@@ -456,8 +456,8 @@ __device__ bool qg_eval_one(const QgEvalArgs& g, const QgTopoDev& tp, const doub
     return true;
 }
 
-template <int T>
-__global__ __launch_bounds__(kThreads) void qg_eval_kernel(QgEvalArgs g) {
+template <int T, int NT>
+__global__ __launch_bounds__(NT) void qg_eval_kernel(QgEvalArgs g) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ int s_inst, s_ok;
     __shared__ int s_passive[64], s_slot[64];
@@ -477,17 +477,17 @@ __global__ __launch_bounds__(kThreads) void qg_eval_kernel(QgEvalArgs g) {
         const double* f = g.fobs + g.inst_fobs[i];
         if (tid < D) s_theta[tid] = g.theta[static_cast<std::int64_t>(i) * g.dmax + tid];
         if (g.mode == 2)
-            for (int e = tid; e < ne; e += kThreads) L.bl[e] = g.bl_in[static_cast<std::int64_t>(i) * g.emax + e];
+            for (int e = tid; e < ne; e += NT) L.bl[e] = g.bl_in[static_cast<std::int64_t>(i) * g.emax + e];
         __syncthreads();
         double* fit = g.fit_out ? g.fit_out + static_cast<std::int64_t>(i) * g.np_max : nullptr;
-        const bool ok = qg_eval_one<T>(g, tp, G, f, g.mode, L, sh, fit);
+        const bool ok = qg_eval_one<T, NT>(g, tp, G, f, g.mode, L, sh, fit);
         if (tid == 0) g.score[i] = s_scal[1];
         if (ok) {
             if (g.bl_out)
-                for (int e = tid; e < ne; e += kThreads) g.bl_out[static_cast<std::int64_t>(i) * g.emax + e] = L.bl[e];
+                for (int e = tid; e < ne; e += NT) g.bl_out[static_cast<std::int64_t>(i) * g.emax + e] = L.bl[e];
             if (g.mode != 0 && tid < D) g.grad_theta[static_cast<std::int64_t>(i) * g.dmax + tid] = s_thbar[tid];
             if (g.mode == 2)
-                for (int e = tid; e < ne; e += kThreads)
+                for (int e = tid; e < ne; e += NT)
                     g.grad_bl[static_cast<std::int64_t>(i) * g.emax + e] = L.blbar[e];
         }
         __syncthreads();
@@ -510,8 +510,8 @@ constexpr int kHist = 8;
 constexpr int kMaxBacktrack = 30;
 constexpr double kArmijo = 1e-4;
 
-template <int T>
-__global__ __launch_bounds__(kThreads) void qg_fit_kernel(QgEvalArgs g, QgFitArgs fa) {
+template <int T, int NT>
+__global__ __launch_bounds__(NT) void qg_fit_kernel(QgEvalArgs g, QgFitArgs fa) {
     extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ int s_inst, s_ok, s_stop, s_acc;
     __shared__ int s_passive[64], s_slot[64];
@@ -541,7 +541,7 @@ __global__ __launch_bounds__(kThreads) void qg_fit_kernel(QgEvalArgs g, QgFitArg
         }
         __syncthreads();
         int iters = 0, status = 0;
-        if (!qg_eval_one<T>(g, tp, G, f, D > 0 ? 1 : 0, L, sh, nullptr)) {
+        if (!qg_eval_one<T, NT>(g, tp, G, f, D > 0 ? 1 : 0, L, sh, nullptr)) {
             status = 1;
         } else if (D > 0) {
             if (tid == 0) {
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(kThreads) void qg_fit_kernel(QgEvalArgs g, QgFitArg
                         s_theta[tid] = xn < 0.0 ? 0.0 : (xn > 1.0 ? 1.0 : xn);
                     }
                     __syncthreads();
-                    const bool ok = qg_eval_one<T>(g, tp, G, f, 1, L, sh, nullptr, true);
+                    const bool ok = qg_eval_one<T, NT>(g, tp, G, f, 1, L, sh, nullptr, true);
                     if (tid == 0) {
                         double dec = 0.0;
                         for (int d = 0; d < D; ++d) dec += s_gx[d] * (s_theta[d] - s_x[d]);
@@ -774,50 +774,64 @@ std::size_t qg_eval_lds_bytes(const QgEvalArgs& a) {
     return n * sizeof(double);
 }
 
-int qg_blocks_per_cu(int T, bool fit, std::size_t lds) {
-    int n = 0;
-    auto q = [&](auto kernel) {
-        if (lds > 64 * 1024)
-            STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        STP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kThreads, lds));
-    };
-    if (T == 32) fit ? q(qg_fit_kernel<32>) : q(qg_eval_kernel<32>);
-    else fit ? q(qg_fit_kernel<64>) : q(qg_eval_kernel<64>);
-    return n > 0 ? n : 1;
+// f(kernel) on the score or fit kernel of bucket T with nt threads a workgroup.
+template <class F>
+static void with_eval_kernel(int T, int nt, F&& f) {
+    if (T == 32) nt == 64 ? f(qg_eval_kernel<32, 64>) : f(qg_eval_kernel<32, kThreads>);
+    else if (T == 64) nt == 64 ? f(qg_eval_kernel<64, 64>) : f(qg_eval_kernel<64, kThreads>);
+    else throw ArgError("qpgraph: unsupported edge-count bucket " + std::to_string(T));
+}
+template <class F>
+static void with_fit_kernel(int T, int nt, F&& f) {
+    if (T == 32) nt == 64 ? f(qg_fit_kernel<32, 64>) : f(qg_fit_kernel<32, kThreads>);
+    else if (T == 64) nt == 64 ? f(qg_fit_kernel<64, 64>) : f(qg_fit_kernel<64, kThreads>);
+    else throw ArgError("qpgraph: unsupported edge-count bucket " + std::to_string(T));
 }
 
-void launch_qg_eval(int T, const QgEvalArgs& a, int n_workgroups, hipStream_t st) {
+QgShape qg_shape(int T, bool fit, const QgEvalArgs& a, int n_cu) {
+    const std::size_t lds = qg_eval_lds_bytes(a);
+    auto per_cu = [&](int nt) {
+        int n = 0;
+        auto q = [&](auto kernel) {
+            if (lds > 64 * 1024)
+                STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+            STP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, nt, lds));
+        };
+        fit ? with_fit_kernel(T, nt, q) : with_eval_kernel(T, nt, q);
+        return n > 0 ? n : 1;
+    };
+    const int wide = per_cu(kThreads), narrow = per_cu(64);
+    // One wavefront an instance when the launch fills the device with the wide workgroups
+    // anyway and at least twice as many narrow ones fit a CU (registers, not LDS, bound them):
+    // most of an evaluation runs on one wavefront or one thread between barriers.
+    // 16,700 restarts of graphs with 10 pairs and 11 edges (a 5-population search): fit and
+    // score kernels 30 -> 21.6 ms, the whole search 62 -> 45 ms.  (Graphs of 8-12 leaves, bound by LDS, keep 256.)
+    const bool one_wave = a.n_inst > wide * n_cu && narrow >= 2 * wide;
+    return {one_wave ? 64 : kThreads, std::min(a.n_inst, (one_wave ? narrow : wide) * n_cu)};
+}
+
+void launch_qg_eval(int T, const QgEvalArgs& a, QgShape shape, hipStream_t st) {
     if (a.n_inst <= 0) return;
     const std::size_t lds = qg_eval_lds_bytes(a);
-    auto go = [&](auto kernel) {
+    with_eval_kernel(T, shape.threads, [&](auto kernel) {
         if (lds > 64 * 1024)
             STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        kernel<<<static_cast<unsigned>(n_workgroups), kThreads, lds, st>>>(a);
-    };
-    switch (T) {
-        case 32: go(qg_eval_kernel<32>); break;
-        case 64: go(qg_eval_kernel<64>); break;
-        default: throw ArgError("qpgraph: unsupported edge-count bucket " + std::to_string(T));
-    }
+        kernel<<<static_cast<unsigned>(shape.workgroups), shape.threads, lds, st>>>(a);
+    });
     STP_LAUNCH_CHECK();
 }
 
-void launch_qg_fit(int T, const QgEvalArgs& a, const QgFitArgs& fa, int n_workgroups, hipStream_t st) {
+void launch_qg_fit(int T, const QgEvalArgs& a, const QgFitArgs& fa, QgShape shape, hipStream_t st) {
     if (a.n_inst <= 0) return;
     const std::size_t lds = qg_eval_lds_bytes(a);
-    auto go = [&](auto kernel) {
+    with_fit_kernel(T, shape.threads, [&](auto kernel) {
         if (lds > 64 * 1024)
             STP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        kernel<<<static_cast<unsigned>(n_workgroups), kThreads, lds, st>>>(a, fa);
-    };
-    switch (T) {
-        case 32: go(qg_fit_kernel<32>); break;
-        case 64: go(qg_fit_kernel<64>); break;
-        default: throw ArgError("qpgraph: unsupported edge-count bucket " + std::to_string(T));
-    }
+        kernel<<<static_cast<unsigned>(shape.workgroups), shape.threads, lds, st>>>(a, fa);
+    });
     STP_LAUNCH_CHECK();
 }
 
