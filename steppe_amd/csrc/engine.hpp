@@ -10,6 +10,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <map>
 #include <memory>
 #include <string>
@@ -431,7 +432,8 @@ private:
     // their sizes and total; then the survivor-transposed tensor in qpT_.
     void survivor_list(const F2Blocks& h, std::vector<std::int32_t>& surv, std::vector<std::int32_t>& bsz,
                        double& n_total);
-    FstatTensor survivor_tensor(const F2Blocks& h, std::vector<std::int32_t>* bsz_out = nullptr);
+    FstatTensor survivor_tensor(const F2Blocks& h, std::vector<std::int32_t>* bsz_out = nullptr,
+                                const std::function<bool(int)>& in_place = {});
     // The Gram form of an f4 sweep (fstats_host.cpp); appends |z| >= tau survivors.
     void f4_sweep_gram(const FstatTensor& t, const std::vector<std::int32_t>& bsz, int range,
                        const std::int32_t* d_subset, const std::vector<std::int64_t>& binom, std::int64_t K,

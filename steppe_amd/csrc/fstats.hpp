@@ -15,6 +15,8 @@ struct FstatTensor {
     const std::int32_t* bsz = nullptr;  // survivor block sizes [nbs]
     int P = 0, nbs = 0;
     double n_total = 0.0;           // sum of the survivor block sizes
+    const double* f2 = nullptr;     // the tensor itself, [i + P*j + P*P*b]
+    const std::int32_t* surv = nullptr;  // surviving blocks [nbs]
 };
 
 // One statistic per wavefront: width 4 (f4 of (p1, p2, p3, p4)) or 3 (f3 of (C; A, B)).
@@ -23,8 +25,11 @@ struct FstatArgs {
     const std::int32_t* idx = nullptr;  // N * width population indices
     std::int64_t N = 0;
     double *est = nullptr, *se = nullptr, *z = nullptr, *p = nullptr;
+    bool direct = false;            // read t.f2 block by block instead of t.f2T
 };
 void launch_fstat(int width, const FstatArgs& a, hipStream_t st);
+// Whether N statistics of a tensor are read block by block rather than from a transposed copy.
+bool fstat_direct(int width, std::int64_t N, int P, int nbs);
 
 // One (p1, p2, p3, p4, p5) tuple per wavefront: alpha = f4(p1,p2;p3,p4) / f4(p1,p2;p5,p4).
 struct F4RatioArgs {

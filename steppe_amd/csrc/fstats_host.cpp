@@ -98,7 +98,8 @@ void HipBackend::survivor_list(const F2Blocks& h, std::vector<std::int32_t>& sur
         }
 }
 
-FstatTensor HipBackend::survivor_tensor(const F2Blocks& h, std::vector<std::int32_t>* bsz_out) {
+FstatTensor HipBackend::survivor_tensor(const F2Blocks& h, std::vector<std::int32_t>* bsz_out,
+                                        const std::function<bool(int)>& in_place) {
     std::vector<std::int32_t> surv, bsz;
     double n_total = 0.0;
     survivor_list(h, surv, bsz, n_total);
@@ -115,8 +116,12 @@ FstatTensor HipBackend::survivor_tensor(const F2Blocks& h, std::vector<std::int3
     STP_HIP(hipMemcpyAsync(fs_i32_.get(), arena.data(), arena.size() * sizeof(std::int32_t), hipMemcpyHostToDevice,
                            stream_));
     const std::int64_t slab = static_cast<std::int64_t>(h.P) * h.P;
-    qpT_.ensure(static_cast<std::size_t>(slab) * t.nbs);
-    launch_transpose_survivors(h.f2.get(), slab, fs_i32_.get(), t.nbs, qpT_.get(), stream_);
+    t.f2 = h.f2.get();
+    t.surv = fs_i32_.get();
+    if (!(in_place && in_place(t.nbs))) {
+        qpT_.ensure(static_cast<std::size_t>(slab) * t.nbs);
+        launch_transpose_survivors(h.f2.get(), slab, fs_i32_.get(), t.nbs, qpT_.get(), stream_);
+    }
     // The arena is pageable host memory that goes out of scope here.
     STP_HIP(hipStreamSynchronize(stream_));
     t.f2T = qpT_.get();
@@ -134,7 +139,8 @@ void HipBackend::fstat(const F2Blocks& h, int width, std::int64_t n, const std::
     for (std::int64_t k = 0; k < n * width; ++k)
         STP_REQUIRE(idx[k] >= 0 && idx[k] < h.P,
                     "fstat: population index out of range in tuple " + std::to_string(k / width));
-    const FstatTensor t = survivor_tensor(h);
+    const auto in_place = [&](int nbs) { return fstat_direct(width, n, h.P, nbs); };
+    const FstatTensor t = survivor_tensor(h, nullptr, in_place);
     if (t.nbs == 0) {
         std::fill(est, est + n, std::nan(""));
         std::fill(se, se + n, std::nan(""));
@@ -154,6 +160,7 @@ void HipBackend::fstat(const F2Blocks& h, int width, std::int64_t n, const std::
     a.se = a.est + n;
     a.z = a.se + n;
     a.p = a.z + n;
+    a.direct = in_place(t.nbs);
     mark_begin(kFstat);
     launch_fstat(width, a, stream_);
     mark_end(kFstat);

@@ -485,8 +485,9 @@ void qpadm_fit_kernel(QpFitArgs g, int n_parts, int refits, int nr_max) {
     const int nl = md.nl, nr = md.nr, m = md.m, nbs = g.nbs, rank = md.rank, ldq = m + 1;
     const QpSetup sp = qp_setup(g.setup, md, nbs);
     const double* wmain = rank == nl - 1 ? tb->wrf[0] : tb->wmain;
-    if (refits && !qpadm_do_se(tb->ok[0][rank] != 0, nbs, g.jackknife, wmain, nl, g.se_require_p != 0,
-                               tb->chisq[0][rank], dof_of(nl, nr, rank), g.p_se_threshold))
+    if (refits &&
+        !qpadm_do_se(tb->ok[0][rank] != 0, nbs, g.jackknife, wmain, nl, g.se_require_p != 0, tb->chisq[0][rank],
+                     dof_of(nl, nr, rank), g.p_se_threshold))
         return;
     const WaveSlice W = slice_at(lds + m * ldq + wave * wave_slice(nr_max), nr_max);
     for (int e = tid; e < m * m; e += kQThreads) {
@@ -593,15 +594,28 @@ __global__ __launch_bounds__(kQThreads) void qpadm_finish_kernel(QpFitArgs g, in
 // ---------------------------------------------------------------------------------
 // keep[b] = !(some pair has vpair <= 0 and another has vpair > 0)
 // (the reference's survivor_blocks, cpu_backend.cpp:125-150).
-__global__ __launch_bounds__(256) void survivor_kernel(const double* __restrict__ vpair, std::int64_t slab,
-                                                       std::int32_t* __restrict__ keep) {
+// Bound by HBM (8 bytes a pair and block): sixteen wavefronts a block with four loads in
+// flight each: 200 populations x 744 blocks (238 MB) 87 -> 47 us = 5.1 TB/s against four
+// wavefronts with one.
+constexpr int kSurvThreads = 1024;
+__global__ __launch_bounds__(kSurvThreads) void survivor_kernel(const double* __restrict__ vpair, std::int64_t slab,
+                                                                std::int32_t* __restrict__ keep) {
     const std::int64_t b = blockIdx.x;
     const double* v = vpair + b * slab;
     int pres = 0, miss = 0;
-    for (std::int64_t e = threadIdx.x; e < slab; e += blockDim.x) {
-        if (v[e] > 0.0) pres = 1;
+    auto see = [&](double x) {
+        if (x > 0.0) pres = 1;
         else miss = 1;
+    };
+    std::int64_t e = threadIdx.x;
+    for (; e + 3 * kSurvThreads < slab; e += 4 * kSurvThreads) {
+        const double x0 = v[e], x1 = v[e + kSurvThreads], x2 = v[e + 2 * kSurvThreads], x3 = v[e + 3 * kSurvThreads];
+        see(x0);
+        see(x1);
+        see(x2);
+        see(x3);
     }
+    for (; e < slab; e += kSurvThreads) see(v[e]);
     pres = __syncthreads_or(pres);
     miss = __syncthreads_or(miss);
     if (threadIdx.x == 0) keep[b] = (pres && miss) ? 0 : 1;
@@ -632,7 +646,7 @@ __global__ __launch_bounds__(256) void transpose_survivors_kernel(const double* 
 
 void launch_survivors(const double* vpair, std::int64_t slab, int n_block, std::int32_t* keep, hipStream_t st) {
     if (n_block <= 0) return;
-    survivor_kernel<<<static_cast<unsigned>(n_block), 256, 0, st>>>(vpair, slab, keep);
+    survivor_kernel<<<static_cast<unsigned>(n_block), kSurvThreads, 0, st>>>(vpair, slab, keep);
     STP_LAUNCH_CHECK();
 }
 
