@@ -128,6 +128,12 @@ HipBackend::~HipBackend() {
         (void)hipStreamSynchronize(stream_);
         (void)hipStreamDestroy(stream_);
     }
+    for (hipEvent_t e : side_ev_)
+        if (e) (void)hipEventDestroy(e);
+    if (side_stream_) {
+        (void)hipStreamSynchronize(side_stream_);
+        (void)hipStreamDestroy(side_stream_);
+    }
 }
 
 void HipBackend::activate() const { STP_HIP(hipSetDevice(device_)); }

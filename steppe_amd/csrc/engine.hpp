@@ -484,6 +484,9 @@ private:
     NoallocScratch noalloc_;   // this device's address of the allocation-free decode's scratch
     std::string name_;
     hipStream_t stream_ = nullptr;
+    hipStream_t side_stream_ = nullptr;   // qpAdm fit tables beside their refits; made at first use
+    hipEvent_t side_ev_[2] = {nullptr, nullptr};
+    hipStream_t side_stream();
 
     // Pooled workspaces (grow-only).
     DevBuf<std::uint8_t> packed_stage_;

@@ -485,7 +485,7 @@ void qpadm_fit_kernel(QpFitArgs g, int n_parts, int refits, int nr_max) {
     const int nl = md.nl, nr = md.nr, m = md.m, nbs = g.nbs, rank = md.rank, ldq = m + 1;
     const QpSetup sp = qp_setup(g.setup, md, nbs);
     const double* wmain = rank == nl - 1 ? tb->wrf[0] : tb->wmain;
-    if (refits &&
+    if (refits && !g.all_refits &&
         !qpadm_do_se(tb->ok[0][rank] != 0, nbs, g.jackknife, wmain, nl, g.se_require_p != 0, tb->chisq[0][rank],
                      dof_of(nl, nr, rank), g.p_se_threshold))
         return;

@@ -97,6 +97,7 @@ struct QpFitArgs {
     int se_require_p = 0;
     double p_se_threshold = 0.05;
     int slot0 = 0;
+    bool all_refits = false;       // refit every model: the fit tables may still be running
 };
 
 // A model's setup results: tau and the leave-one-out values [m][nbs], Qinv [m][m], totals.

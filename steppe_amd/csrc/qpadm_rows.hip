@@ -494,8 +494,8 @@ void qpadm_rows_kernel(QpFitArgs g, int n_parts) {
     if (!tb->cov_ok) return;
     const int nr = __builtin_amdgcn_readfirstlane(md.nr), m = NL * nr, nbs = g.nbs;
     const double* wmain = md.rank == NL - 1 ? tb->wrf[0] : tb->wmain;
-    if (!qpadm_do_se(tb->ok[0][md.rank] != 0, nbs, g.jackknife, wmain, NL, g.se_require_p != 0,
-                     tb->chisq[0][md.rank], dof_of(NL, nr, md.rank), g.p_se_threshold))
+    if (!g.all_refits && !qpadm_do_se(tb->ok[0][md.rank] != 0, nbs, g.jackknife, wmain, NL, g.se_require_p != 0,
+                                      tb->chisq[0][md.rank], dof_of(NL, nr, md.rank), g.p_se_threshold))
         return;
     const QpSetup sp = qp_setup(g.setup, md, nbs);
     const int ldq = m | 1;
