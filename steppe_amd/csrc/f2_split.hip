@@ -435,13 +435,15 @@ __device__ inline i4 v_of_w0(i4 w0) {
     return __builtin_bit_cast(i4, x);
 }
 
-// s_waitcnt on the vector-memory count only (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14; expcnt 6:4 and lgkmcnt 11:8 left at their maxima).  As a builtin, unlike
-// inline assembly, the compiler's wait-count tracking takes it into account.
+// s_waitcnt on the vector-memory count and, to zero, on this wavefront's LDS reads (gfx9
+// encoding: vmcnt in bits 3:0 and 15:14, lgkmcnt 11:8; expcnt 6:4 left at its maximum): at a
+// phase barrier no read of the slot that is refilled next may still be under way, wherever
+// the compiler put the products that use it.  As a builtin, unlike inline assembly, the
+// compiler's wait-count tracking takes it into account.
 template <int N>
 __device__ inline void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "vmcnt is six bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
 }
 
 // Issue this wavefront's share of one slot's 1 KB chunks (direct global->LDS): chunk
