@@ -24,8 +24,8 @@ FP64" configuration).
 
 Extra JSON fields: ``roofline`` for the dominant kernel (the f2 contraction),
 timed with HIP events on the engine's own stream: achieved = k * F_alg / t, with
-F_alg = 8 W FLOP (4 MACs per pair-SNP) and k = 1 for the FP64 form, k = 7.25 for the
-split form (29 BF16/FP16 MFMA products per pair-SNP over 4 MACs); ``traffic`` is the HBM bytes
+F_alg = 8 W FLOP (4 MACs per pair-SNP) and k = 1 for the FP64 form, k = 8.25 for the
+split form (33 int8 MFMA products per pair-SNP over 4 MACs, against the int8 peak); ``traffic`` is the HBM bytes
 per launch from the committed rocprofv3 counter summary of the same workload
 (profiles/), or null; ``stages`` with every stage's average device time;
 ``cpu_baseline``: the reference CpuBackend (oracle/_ref, compiled from the reference
@@ -64,8 +64,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 SEED = 20261202
-MI355X_PEAK = {"hbm_GBs": 8000.0, "fp64_TFLOPs": 78.6, "bf16_TFLOPs": 2500.0}
-SPLIT_K = 29 * 2 / 8.0   # executed BF16/FP16 MFMA FLOP per algorithmic FLOP in the split form
+MI355X_PEAK = {"hbm_GBs": 8000.0, "fp64_TFLOPs": 78.6, "int8_TOPs": 5000.0}
+SPLIT_K = 33 * 2 / 8.0   # executed int8 MFMA operations per algorithmic FLOP in the split form
 PROFILES = {("c3", "split_bf16"): ("profiles/f2_split_c3.md", "f2_split_kernel", "f2_split.hip"),
             ("c3", "fp64"): ("profiles/f2_fp64_c3.md", "f2_fp64_kernel", "f2_fp64.hip")}
 METRIC = "f2 pop-pair·SNPs/sec at ≤1e-9 rel err (split-BF16 vs FP64); qpAdm fits/sec"
@@ -770,17 +770,17 @@ def main():
     f_alg = 8.0 * W
     f2_s = avg["f2"] / 1e3
     fp64 = prec == _core.STP_PREC_FP64
-    peak = MI355X_PEAK["fp64_TFLOPs"] if fp64 else MI355X_PEAK["bf16_TFLOPs"]
+    peak = MI355X_PEAK["fp64_TFLOPs"] if fp64 else MI355X_PEAK["int8_TOPs"]
     kf = 1.0 if fp64 else SPLIT_K
     achieved = kf * f_alg / f2_s / 1e12 if f2_s > 0 else 0.0
     traffic, traffic_src = profiled_traffic(args.workload, args.precision)
     roofline = {"kernel": "f2_fp64_kernel" if fp64 else "f2_split_kernel",
-                "bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+                "bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s" if fp64 else "TOP/s",
                 "frac": achieved / peak, "traffic": traffic, "traffic_source": traffic_src,
                 "k": kf, "algorithmic_TFLOPs": f_alg / f2_s / 1e12 if f2_s > 0 else 0.0,
                 "work": ("8*W FLOP per launch, W = P(P+1)/2*M" if fp64 else
-                         "k*8*W FLOP per launch (k = 7.25 BF16/FP16 MFMA FLOP per algorithmic FLOP: 21 BF16 "
-                         "digit products + 8 FP16 w-digit x V products per pair-SNP), W = P(P+1)/2*M")}
+                         "k*8*W operations per launch (k = 8.25 int8 MFMA operations per algorithmic FLOP: 21 "
+                         "digit products + 12 w-digit x V products per pair-SNP), W = P(P+1)/2*M")}
     dec_bytes = n_ind * bpr + 4 * P * M
     stages = {k: {"avg_ms": avg[k]} for k in avg}
     stages["decode"]["hbm_GBs"] = dec_bytes / (avg["decode"] / 1e3) / 1e9 if avg["decode"] else None
@@ -871,7 +871,7 @@ def main():
         "metric": METRIC, "value": value, "unit": "pop-pair·SNPs/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": ms_step,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f64" if prec == _core.STP_PREC_FP64 else "bf16x(split)->f64",
+        "dtype": "f64" if prec == _core.STP_PREC_FP64 else "int8x6 (48-bit fixed point)->f64",
         "data": "synthetic (Balding-Nichols panel generated in HBM)",
         "config": {"workload": f"{args.workload}: {P} populations x {M} SNPs, {n_ind} individuals, "
                                f"{nb} jackknife blocks, decode + f2 ({args.precision})",
