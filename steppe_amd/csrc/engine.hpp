@@ -525,6 +525,7 @@ private:
     DevBuf<std::int64_t> fs_i64_;
     DevBuf<SweepHit> fs_hits_, fs_select_;
     DevBuf<unsigned> fs_hist_;
+    DevBuf<double> fs_table_;
     DevBuf<unsigned long long> fs_count_;
     DevBuf<double> fs_mean_, fs_wroot_;
     DevBuf<GramItem> fs_items_;

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 namespace stp {
@@ -17,7 +18,13 @@ struct FstatTensor {
     double n_total = 0.0;           // sum of the survivor block sizes
     const double* f2 = nullptr;     // the tensor itself, [i + P*j + P*P*b]
     const std::int32_t* surv = nullptr;  // surviving blocks [nbs]
+    // what the jackknife of any series needs of the block sizes (launch_block_table):
+    // rel = size / n, w = 1 - rel, h = n / size, sqrt(h - 1), each [nbs], then the
+    // double-double sum of w
+    const double* table = nullptr;
 };
+inline std::size_t block_table_doubles(int nbs) { return 4 * static_cast<std::size_t>(nbs) + 2; }
+void launch_block_table(const FstatTensor& t, double* table, hipStream_t st);
 
 // One statistic per wavefront: width 4 (f4 of (p1, p2, p3, p4)) or 3 (f3 of (C; A, B)).
 struct FstatArgs {

@@ -162,6 +162,11 @@ void HipBackend::fstat(const F2Blocks& h, int width, std::int64_t n, const std::
     a.p = a.z + n;
     a.direct = in_place(t.nbs);
     mark_begin(kFstat);
+    if (!a.direct) {
+        fs_table_.ensure(block_table_doubles(t.nbs));
+        launch_block_table(t, fs_table_.get(), stream_);
+        a.t.table = fs_table_.get();
+    }
     launch_fstat(width, a, stream_);
     mark_end(kFstat);
     std::vector<double> host(static_cast<std::size_t>(4) * n);
