@@ -15,14 +15,13 @@
 // lockstep so that each round's unscored neighbours are fitted in one fleet.
 #include <chrono>
 #include <cmath>
-#include <functional>
-#include <future>
 #include <limits>
 #include <memory>
 #include <unordered_map>
 #include <unordered_set>
 
 #include "engine.hpp"
+#include "host_pool.hpp"
 #include "qpgraph.hpp"
 #include "qpgraph_enum.hpp"
 
@@ -222,20 +221,16 @@ QgSearchResult HipBackend::qpgraph_search(const F2Blocks& f2, const std::vector<
         for (int step = 0; step < kMaxClimbSteps; ++step) {
             std::vector<std::vector<qgenum::Candidate>> nb(K);
             want.clear();
-            bool any = false;
-            // the seeds' moves in parallel (a future hands an exception on to this thread)
-            std::vector<std::future<std::vector<qgenum::Candidate>>> moves(K);
+            // the seeds' moves in parallel: their number is the caller's choice, the threads' is not
+            std::vector<int> climbing;
             for (int k = 0; k < K; ++k)
-                if (active[k])
-                    moves[k] = std::async(std::launch::async, qgenum::neighbors, std::cref(cur[k]), std::cref(pops),
-                                          max_nadmix);
-            for (int k = 0; k < K; ++k) {
-                if (!active[k]) continue;
-                any = true;
-                nb[k] = moves[k].get();
+                if (active[k]) climbing.push_back(k);
+            if (climbing.empty()) break;
+            for_each_index(climbing.size(), [&](std::size_t i) {
+                nb[climbing[i]] = qgenum::neighbors(cur[climbing[i]], pops, max_nadmix);
+            });
+            for (int k : climbing)
                 for (const auto& c : nb[k]) want.push_back(&c);
-            }
-            if (!any) break;
             score_missing(want);
             for (int k = 0; k < K; ++k) {
                 if (!active[k]) continue;

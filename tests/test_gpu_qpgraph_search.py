@@ -115,3 +115,50 @@ def test_errors(handle):
         qg.run_qpgraph_search(handle, ["Mbuti", "Han", "Nowhere"])
     with pytest.raises(ValueError, match="twice"):
         qg.run_qpgraph_search(handle, ["Mbuti", "Han", "Mbuti"])
+
+
+def _serial_climb(search, n_seeds):
+    """The hill-climb one seed at a time, from the candidates' scores."""
+    c = search["cands"]
+    score = search["score"]
+    moves = search["moves"]
+    out = []
+    for k in range(n_seeds):
+        cur = c[k * len(c) // n_seeds]
+        for _ in range(1000):
+            key = tuple(map(tuple, cur["edges"]))   # two wirings of one shape have different base trees
+            if key not in moves:
+                moves[key] = qg.topology_neighbors(cur, POPS, 1)
+            nb = moves[key]
+            best = min(nb, key=lambda g: score[g["hash"]])    # the first of equal scores
+            if not score[best["hash"]] < score[cur["hash"]]:
+                break
+            cur = best
+        out.append(cur["hash"])
+    return out
+
+
+@pytest.mark.parametrize("n_seeds", [40, 300])
+def test_more_seeds_than_threads(search, handle, n_seeds):
+    # any number of seeds climbs on a bounded number of threads, to the serial climb's graphs
+    import threading
+    base = len(os.listdir("/proc/self/task"))
+    peak, stop = [0], threading.Event()
+
+    def watch():
+        while not stop.wait(0.0005):
+            peak[0] = max(peak[0], len(os.listdir("/proc/self/task")))
+
+    w = threading.Thread(target=watch)
+    w.start()
+    try:
+        d = qg.run_qpgraph_search(handle, POPS, heuristic_seeds=n_seeds)
+    finally:
+        stop.set()
+        w.join()
+    assert d["cand_score"] == search["cand_score"] and len(d["seed_hashes"]) == n_seeds
+    extra = peak[0] - base - 1
+    _say(f"{n_seeds} seeds: at most {extra} threads beside the caller's")
+    assert extra < 32                      # 15 of the climb, the rest for the runtime's own
+    state = {"cands": qg.enumerate_graphs(POPS, 1), "score": dict(zip(d["cand_hash"], d["cand_score"])), "moves": {}}
+    assert d["seed_hashes"] == _serial_climb(state, n_seeds)
