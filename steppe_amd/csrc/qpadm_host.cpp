@@ -236,7 +236,7 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
 // refit weights fit a fixed budget; per chunk the models are ordered by kernel instance and
 // each stage is one launch per instance.
 void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, const stp_qpadm_options& opt) {
-    constexpr std::size_t kSetupBudget = std::size_t{1} << 29;   // doubles (4 GiB)
+    constexpr std::size_t kBudget = std::size_t{1} << 29;        // doubles (4 GiB): setup results and weights
     constexpr std::size_t kMaxChunk = 16384;                     // models
     const int nbs = a.nbs;
     auto cls = [&](const QpLargeModel& md) {
@@ -250,13 +250,14 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
         return x.m > y.m;
     });
     const bool refits = a.jackknife != 0 && nbs >= 2;
+    const std::size_t weights = refits ? static_cast<std::size_t>(STP_QPADM_MAX_NL) * nbs : 0;   // of a model
     for (std::size_t i0 = 0; i0 < models.size();) {
         std::size_t setup = 0, i1 = i0;
         int m_max = 0;
         for (; i1 < models.size() && i1 - i0 < kMaxChunk; ++i1) {
             QpLargeModel& md = models[i1];
-            const std::size_t need = qp_setup_doubles(md.m, nbs) + (refits ? STP_QPADM_MAX_NL * nbs : 0);
-            if (i1 > i0 && setup + need > kSetupBudget) break;
+            const std::size_t need = qp_setup_doubles(md.m, nbs);
+            if (i1 > i0 && setup + need + (i1 - i0 + 1) * weights > kBudget) break;
             md.base = static_cast<std::int64_t>(setup);
             setup += need;
             m_max = std::max(m_max, md.m);
@@ -273,7 +274,7 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
         a.tables = ql_tables_.get();
         a.setup = ql_setup_.get();
         if (refits) {
-            ql_wm_.ensure(static_cast<std::size_t>(nm) * nbs * STP_QPADM_MAX_NL);
+            ql_wm_.ensure(nm * weights);
             a.wm = ql_wm_.get();
         }
         launch_qpadm_setup(a, nm, m_max, stream_);
