@@ -9,9 +9,11 @@
 // order.  The f2 slab is first transposed to pair-major, survivor-only order so a
 // model's f4 basis reads each f2 series contiguously.
 #include <algorithm>
+#include <cstdlib>
 #include <numeric>
 #include <vector>
 
+#include "chunks.hpp"
 #include "engine.hpp"
 #include "qpadm.hpp"
 
@@ -233,8 +235,8 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
 }
 
 // Models whose fits hold a matrix row per lane: chunks of models whose setup results and
-// refit weights fit a fixed budget; per chunk the models are ordered by kernel instance and
-// each stage is one launch per instance.
+// refit weights fit a fixed budget, or what is free beside a large resident tensor; per chunk
+// the models are ordered by kernel instance and each stage is one launch per instance.
 void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, const stp_qpadm_options& opt) {
     constexpr std::size_t kBudget = std::size_t{1} << 29;        // doubles (4 GiB): setup results and weights
     constexpr std::size_t kMaxChunk = 16384;                     // models
@@ -251,21 +253,37 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
     });
     const bool refits = a.jackknife != 0 && nbs >= 2;
     const std::size_t weights = refits ? static_cast<std::size_t>(STP_QPADM_MAX_NL) * nbs : 0;   // of a model
-    for (std::size_t i0 = 0; i0 < models.size();) {
-        std::size_t setup = 0, i1 = i0;
-        int m_max = 0;
-        for (; i1 < models.size() && i1 - i0 < kMaxChunk; ++i1) {
-            QpLargeModel& md = models[i1];
-            const std::size_t need = qp_setup_doubles(md.m, nbs);
-            if (i1 > i0 && setup + need + (i1 - i0 + 1) * weights > kBudget) break;
-            md.base = static_cast<std::int64_t>(setup);
-            setup += need;
-            m_max = std::max(m_max, md.m);
+    // Models per chunk; STEPPE_QPADM_CHUNK lowers it (tests).
+    std::size_t max_chunk = kMaxChunk;
+    if (const char* env = std::getenv("STEPPE_QPADM_CHUNK")) {
+        const long long v = std::strtoll(env, nullptr, 10);
+        if (v > 0) max_chunk = std::min<std::size_t>(max_chunk, static_cast<std::size_t>(v));
+    }
+    int m_max = 0;   // of the chunk
+    auto reserve = [&](std::size_t i0, std::size_t i1) {
+        std::size_t setup = 0;
+        m_max = 0;
+        for (std::size_t i = i0; i < i1; ++i) {
+            models[i].base = static_cast<std::int64_t>(setup);
+            setup += qp_setup_doubles(models[i].m, nbs);
+            m_max = std::max(m_max, models[i].m);
         }
+        try {
+            ql_models_.ensure(i1 - i0);
+            ql_tables_.ensure(i1 - i0);
+            ql_setup_.ensure(setup);
+            ql_wm_.ensure((i1 - i0) * weights);
+        } catch (const OomError&) {
+            if (i1 - i0 == 1) throw;
+            (void)hipGetLastError();   // or the next launch's check would report it
+            ql_setup_.release();
+            ql_wm_.release();
+            return false;
+        }
+        return true;
+    };
+    auto run = [&](std::size_t i0, std::size_t i1) {
         const int nm = static_cast<int>(i1 - i0);
-        ql_models_.ensure(nm);
-        ql_tables_.ensure(nm);
-        ql_setup_.ensure(setup);
         STP_HIP(hipMemcpyAsync(ql_models_.get(), models.data() + i0, nm * sizeof(QpLargeModel), hipMemcpyHostToDevice,
                                stream_));
         launch_zero_u32(reinterpret_cast<unsigned*>(ql_tables_.get()),
@@ -273,10 +291,7 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
         a.models = ql_models_.get();
         a.tables = ql_tables_.get();
         a.setup = ql_setup_.get();
-        if (refits) {
-            ql_wm_.ensure(nm * weights);
-            a.wm = ql_wm_.get();
-        }
+        a.wm = ql_wm_.get();
         launch_qpadm_setup(a, nm, m_max, stream_);
         // runs of models that share a kernel instance
         auto runs = [&](auto key, auto launch) {
@@ -311,10 +326,11 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
                  });
         beside.join();
         launch_qpadm_finish(a, nm, opt.rank_alpha, qp_out_.get(), stream_);
-        if (i1 < models.size()) sync();   // the next chunk reuses the buffers' host copies
-        i0 = i1;
-    }
-    sync();   // the models (host memory) must outlive their copy
+        sync();   // the models (host memory) must outlive their copy, the buffers this chunk
+    };
+    for_chunks(
+        models.size(), max_chunk, kBudget,
+        [&](std::size_t i) { return qp_setup_doubles(models[i].m, nbs) + weights; }, reserve, run);
 }
 
 // Models beyond the batched kernel: chunks of models whose setup scratch fits a fixed

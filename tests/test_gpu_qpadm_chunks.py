@@ -32,3 +32,33 @@ def test_memory_of_a_fleet():
     print(f"{n} models: {grown / 2 ** 20:.0f} MiB more, {kept / 2 ** 20:.0f} MiB of results", flush=True)
     # beside them a fit table, a model and a record each (under 8 KiB) and allocation granules
     assert grown <= kept + 8192 * n + (16 << 20)
+
+
+def _mixed(n, P, seed=4):
+    """Models of every refit kernel: 1-5 sources in the row form's instances, 6-7 sources and
+    more right populations with a wavefront a fit, and one beyond 64 entries."""
+    rng = np.random.default_rng(seed)
+    shapes = [(1, 3), (2, 2), (2, 9), (2, 14), (3, 5), (3, 11), (3, 16), (4, 8), (4, 12), (5, 6), (5, 12), (6, 7),
+              (7, 9), (2, 20), (6, 12)]
+    out = []
+    for i in range(n):
+        nl, nr = shapes[i % len(shapes)]
+        p = [int(x) for x in rng.permutation(P)]
+        out.append((p[0], p[1:1 + nl], p[1 + nl:2 + nl + nr]))
+    return out
+
+
+@pytest.mark.parametrize("jackknife", ["all", "feasible", "none"])
+def test_chunks_give_the_same_fits(monkeypatch, jackknife):
+    # a call cut into chunks re-uses every workspace: the records are the uncut call's bytes
+    from steppe_amd import _core
+    f2, bs = _tensor(30, 45)
+    h = _core.upload_f2(f2, None, bs, [f"p{i}" for i in range(30)])
+    models = _mixed(47, 30)
+    monkeypatch.delenv("STEPPE_QPADM_CHUNK", raising=False)
+    whole = [bytes(r) for r in _core.qpadm_models(h, models, jackknife=jackknife, raw=True)]
+    assert len({r for r in whole}) == len(models)
+    for chunk in (1, 7, 23, 46):
+        monkeypatch.setenv("STEPPE_QPADM_CHUNK", str(chunk))
+        got = [bytes(r) for r in _core.qpadm_models(h, models, jackknife=jackknife, raw=True)]
+        assert got == whole, chunk
