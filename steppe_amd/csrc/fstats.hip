@@ -505,7 +505,7 @@ __global__ __launch_bounds__(kThreads) void sweep_compact_kernel(SweepSelect a) 
     for (std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < a.n; i += step) {
         unsigned long long slot;
         bool ok;
-        wave_append(sweep_bin(a.hits[i].z) >= cut, a.n_out, a.n, lane_id(), slot, ok);
+        wave_append(sweep_bin(a.hits[i].z) >= cut, a.n_out, a.room, lane_id(), slot, ok);
         if (ok) a.out[slot] = a.hits[i];
     }
 }

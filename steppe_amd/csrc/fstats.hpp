@@ -71,16 +71,18 @@ void launch_sweep_direct(const SweepArgs& a, hipStream_t st);
 
 // Selection of a launch's strongest hits on the device: hist counts hits by the top 16 bits
 // of |z| (kSweepBins bins in increasing |z|, each about 6% wide), cut finds the highest bin
-// with at least `keep` hits at or above it, compact copies those hits.  The K strongest hits
-// are among them for every K <= keep.
+// with at least `keep` hits at or above it, compact counts those hits and copies as many of
+// them as out holds.  If it holds them all, the K strongest hits are among them for every
+// K <= keep.
 constexpr int kSweepBins = 1 << 15;
 struct SweepSelect {
     const SweepHit* hits = nullptr;
     std::int64_t n = 0;                     // hits in the buffer
     std::int64_t keep = 0;
     unsigned* hist = nullptr;               // kSweepBins, zeroed by the launch
-    unsigned long long* n_out = nullptr;    // [0] hits selected, [1] the cut bin
-    SweepHit* out = nullptr;                // room for n hits
+    unsigned long long* n_out = nullptr;    // [0] hits selected (of which out holds room), [1] the cut bin
+    SweepHit* out = nullptr;
+    std::int64_t room = 0;                  // hits that out holds
 };
 void launch_sweep_select(const SweepSelect& a, hipStream_t st);
 

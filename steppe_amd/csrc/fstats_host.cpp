@@ -217,14 +217,19 @@ void HipBackend::f4ratio(const F2Blocks& h, std::int64_t n, const std::int32_t* 
 }
 
 // Appends a launch's hits (fs_hits_[0 .. n)) to res; when the sweep keeps far fewer than
-// there are, only the strongest, selected on the device.
+// there are, only the strongest, selected on the device.  The selection overshoots K by the
+// rest of the bin that the K-th hit falls into, 6% of |z|: room for 2 K of them and some more
+// holds it, and where it does not (thousands of statistics with the same |z|) all hits are
+// copied, as for a launch of few.
 void HipBackend::fetch_hits(std::int64_t n, std::int64_t K, std::vector<SweepHit>& res) {
     // Below twice K (or a copy of a megabyte) the selection's three small launches and second
     // synchronisation cost more than the copy that they save.
     constexpr std::int64_t kCopyAll = 1 << 15;
+    constexpr std::int64_t kSelectSpare = 1 << 12;
     const SweepHit* from = fs_hits_.get();
     if (n > std::max(2 * K, kCopyAll)) {
-        fs_select_.ensure(static_cast<std::size_t>(n));
+        const std::int64_t room = std::min<std::int64_t>(n, 2 * K + kSelectSpare);
+        fs_select_.ensure(static_cast<std::size_t>(room));
         fs_hist_.ensure(kSweepBins + 4);
         SweepSelect a;
         a.hits = fs_hits_.get();
@@ -233,14 +238,17 @@ void HipBackend::fetch_hits(std::int64_t n, std::int64_t K, std::vector<SweepHit
         a.hist = fs_hist_.get();
         a.n_out = reinterpret_cast<unsigned long long*>(fs_hist_.get() + kSweepBins);
         a.out = fs_select_.get();
+        a.room = room;
         launch_sweep_select(a, stream_);
         unsigned long long got = 0;
         STP_HIP(hipMemcpyAsync(&got, a.n_out, sizeof(got), hipMemcpyDeviceToHost, stream_));
         STP_HIP(hipStreamSynchronize(stream_));
         STP_REQUIRE(got >= static_cast<unsigned long long>(K) && got <= static_cast<unsigned long long>(n),
                     "fstat_sweep: hit selection out of range");
-        n = static_cast<std::int64_t>(got);
-        from = fs_select_.get();
+        if (got <= static_cast<unsigned long long>(room)) {
+            n = static_cast<std::int64_t>(got);
+            from = fs_select_.get();
+        }
     }
     const std::size_t at = res.size();
     res.resize(at + static_cast<std::size_t>(n));

@@ -5,6 +5,7 @@ import math
 
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +45,43 @@ def test_selection_across_launches(monkeypatch):
     d = _core.run_fstat_sweep(h, 3, min_z=0.0, top_k=500, method="direct")
     for f in FIELDS:
         assert np.array_equal(d[f], whole[f]), f
+
+
+def _four_kinds(P=64, nb=40, seed=9):
+    """Copies of four populations, 16 of each: the 65,536 quartets with one of each kind share
+    three values of |z|, to rounding."""
+    from steppe_amd import _core
+    rng = np.random.default_rng(seed)
+    q = rng.random((4, 1, 60)) * 0.8 + 0.1 + 0.05 * rng.standard_normal((4, nb, 60))
+    q = q[rng.permutation(np.arange(P) % 4)]
+    f2 = np.asfortranarray(((q[:, None] - q[None]) ** 2).mean(-1))
+    return _core.upload_f2(f2, None, rng.integers(50, 90, nb).astype(np.int32), [f"p{i:03d}" for i in range(P)])
+
+
+@pytest.mark.parametrize("method", ["gram", "direct"])
+def test_more_equal_hits_than_the_selection_holds(method):
+    from steppe_amd import _core
+    h = _four_kinds()
+    total = math.comb(64, 4)
+    whole = _core.run_fstat_sweep(h, 4, min_z=0.0, top_k=total, method=method)
+    az = np.abs(whole["z"])
+    for top_k in (1, 100, 1500):
+        # hits of the K-th hit's bin and above: more than 2 K and the spare 4096
+        assert (az >= az[top_k - 1] * (1 - 1e-9)).sum() > 2 * top_k + 4096
+        d = _core.run_fstat_sweep(h, 4, min_z=0.0, top_k=top_k, method=method)
+        for f in FIELDS:
+            assert np.array_equal(d[f], whole[f][:top_k]), (f, top_k)
+
+
+def test_selection_memory():
+    # a sweep's memory follows from its hits; the selection adds what is kept, not all hits again
+    from steppe_amd import _core
+    h = _handle(100)
+    total = math.comb(100, 4)
+    assert len(_core.run_fstat_sweep(h, 4, min_z=1e9)["z"]) == 0     # room for every hit, none found
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    assert len(_core.run_fstat_sweep(h, 4, min_z=0.0, top_k=100)["z"]) == 100
+    grown = before - torch.cuda.mem_get_info()[0]
+    print(f"{total} hits of 32 bytes, 100 kept: {grown / 2 ** 20:.1f} MiB more", flush=True)
+    assert grown <= 8 << 20
