@@ -7,9 +7,8 @@
 // configuration (F2Tune) that the plan carries: the work-item schedule over the dies,
 // the FP64 kernel's wavefront tile (64 x 64 or 32 x 64 outputs), whether it prefetches
 // the next K-step, the FP64 and pair-count grids.  The split kernel's tile is fixed by
-// its LDS ring (one 128 x 128 workgroup per CU); its schedule, the count grid and the order
-// of its LDS reads (the compiler's, or each left fragment one product group ahead) are
-// tuned.  f2_autotune times every candidate on the caller's device inputs (every
+// its LDS ring (one 128 x 128 workgroup per CU); its schedule and the count grid are tuned.
+// f2_autotune times every candidate on the caller's device inputs (every
 // candidate writes bit-identical tensors: the same sums per entry, in the same order),
 // keeps the fastest per key — device name, precision, P, and the block-size histogram
 // (blocks per power-of-two padded length) — and saves the table to a text file
@@ -32,13 +31,13 @@ namespace stp {
 std::string F2Tune::str() const {
     std::ostringstream o;
     o << "sched=" << sched << ",fp64_rows=" << fp64_rows << ",fp64_prefetch=" << fp64_prefetch
-      << ",fp64_wg=" << fp64_wg_per_cu << ",count_wg=" << count_wg_per_cu << ",split_ring=" << split_ring;
+      << ",fp64_wg=" << fp64_wg_per_cu << ",count_wg=" << count_wg_per_cu << ",split_ring=0";
     return o.str();
 }
 
 bool F2Tune::parse(const std::string& s, F2Tune& out) {
     F2Tune t;
-    int found = 0;
+    int found = 0, ring = 0;
     std::stringstream ss(s);
     std::string kv;
     while (std::getline(ss, kv, ',')) {
@@ -51,11 +50,12 @@ bool F2Tune::parse(const std::string& s, F2Tune& out) {
         else if (k == "fp64_prefetch") t.fp64_prefetch = v;
         else if (k == "fp64_wg") t.fp64_wg_per_cu = v;
         else if (k == "count_wg") t.count_wg_per_cu = v;
-        else if (k == "split_ring") t.split_ring = v;
+        else if (k == "split_ring") ring = v;
         else return false;
         ++found;
     }
-    if (found != 6 || (t.split_ring != 0 && t.split_ring != 1) || (t.sched != 0 && t.sched != 1) || (t.fp64_rows != 64 && t.fp64_rows != 32) ||
+    if (found != 6 || (ring != 0 && ring != 1) || (t.sched != 0 && t.sched != 1) ||
+        (t.fp64_rows != 64 && t.fp64_rows != 32) ||
         t.fp64_wg_per_cu < 1 || t.fp64_wg_per_cu > 8 || t.count_wg_per_cu < 1 || t.count_wg_per_cu > 8)
         return false;
     out = t;
@@ -77,15 +77,13 @@ std::string cache_path() {
 std::vector<F2Tune> candidates(int precision) {
     std::vector<F2Tune> c;
     if (precision == STP_PREC_SPLIT_BF16) {
-        for (int ring : {0, 1})
-            for (int sched : {0, 1})
-                for (int cw : {2, 1, 4}) {
-                    F2Tune t;
-                    t.sched = sched;
-                    t.count_wg_per_cu = cw;
-                    t.split_ring = ring;
-                    c.push_back(t);
-                }
+        for (int sched : {0, 1})
+            for (int cw : {2, 1, 4}) {
+                F2Tune t;
+                t.sched = sched;
+                t.count_wg_per_cu = cw;
+                c.push_back(t);
+            }
     } else {
         for (int sched : {0, 1})
             for (int rows : {64, 32})

@@ -432,8 +432,7 @@ void HipBackend::run_f2(const F2Plan& plan, int precision, const F2Source& src, 
     mark_begin(kF2);
     launch_f2_split(w.planeSplit.get(), bt, w.plan.items128.get(), plan.q128, w.counters.get() + kXcds, plan.P,
                     plan.G32, KS32, d_vpair, d_f2, fl,
-                    static_cast<int>(round_up(std::max(1, std::min(n_cu_, n_items128)), kXcds)), tn.split_ring,
-                    stream_);
+                    static_cast<int>(round_up(std::max(1, std::min(n_cu_, n_items128)), kXcds)), stream_);
     mark_end(kF2);
     run_fixup(plan, src, fl, d_f2, d_vpair, w);
 }

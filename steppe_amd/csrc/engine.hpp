@@ -64,7 +64,7 @@ void launch_count_v8(const std::uint8_t* v8, BlockTable bt, const F2Item* items,
                      hipStream_t st);
 void launch_f2_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
                      unsigned* counters, int P, int G32, std::int64_t KS32, const double* vpair, double* f2,
-                     const FixupList& fl, int n_workgroups, int ring, hipStream_t st);
+                     const FixupList& fl, int n_workgroups, hipStream_t st);
 void launch_f2_fixup_counts(const std::uint16_t* a2, const std::uint16_t* n, std::int64_t ld, BlockTable bt,
                             const FixupList& fl, int P, int n_block, const double* vpair, double* f2,
                             int n_workgroups, hipStream_t st);
@@ -100,8 +100,8 @@ struct F2Tune {
     int fp64_prefetch = 1;    // FP64: load the next K-step while this one's MFMAs run
     int fp64_wg_per_cu = 2;   // FP64 contraction workgroups (4 wavefronts) per CU
     int count_wg_per_cu = 2;  // pair-count kernel workgroups per CU
-    int split_ring = 0;       // split contraction's reads of its LDS ring: 0 in the compiler's
-                              // order, 1 each left fragment one product group ahead
+    // The saved text has one more field, split_ring, of a variant that is gone: written as 0,
+    // read as 0 or 1 from tables of earlier versions, without effect.
     std::string str() const;
     static bool parse(const std::string& s, F2Tune& out);
 };

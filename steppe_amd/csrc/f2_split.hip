@@ -462,9 +462,11 @@ __device__ inline void stage_slot(const std::uint8_t* const (&src)[kSetPlanes], 
 }
 
 // The products of one phase for the wavefront's NX sub-tiles: left groups li .. li + NX - 1
-// against right group rj of a slot.
+// against right group rj of a slot.  Where the LDS reads stand is the compiler's choice: with
+// each left fragment read one product group ahead, extractions of 10 to 1000 populations were
+// as fast at best and up to 4% slower.
 template <int NX>
-__device__ __forceinline__ void mul_q_c(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+__device__ __forceinline__ void mul_q(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
     i4 dj[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) dj[k] = lds_frag(slot, rj, k, lane);
@@ -481,7 +483,7 @@ __device__ __forceinline__ void mul_q_c(i16v (&L)[NX][6], const std::uint8_t* sl
 }
 
 template <int NX>
-__device__ __forceinline__ void mul_w_c(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
+__device__ __forceinline__ void mul_w(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
     i4 wj[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) wj[k] = lds_frag(slot, rj, k, lane);
@@ -500,51 +502,6 @@ __device__ __forceinline__ void mul_w_c(i16v (&L)[NX][6], const std::uint8_t* sl
     }
 }
 
-// The same with each left fragment read from LDS one product group ahead of its use (the
-// compiler otherwise reads it right before).  The tuner chooses: 9.22 ms (compiler's order)
-// against 9.42 ms at 1000 populations x 600k SNPs, 1.27 against 1.32 ms at 200 x 1.2M.
-template <int NX>
-__device__ __forceinline__ void mul_q_a(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
-    i4 dj[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) dj[k] = lds_frag(slot, rj, k, lane);
-    i4 di = lds_frag(slot, li, 0, lane);
-    static_for<6 * NX>([&](auto ic) {
-        constexpr int i = decltype(ic)::value, k = i / NX, x = i % NX;
-        constexpr int kn = (i + 1) / NX, xn = (i + 1) % NX;
-        i4 nx = di;
-        if constexpr (i + 1 < 6 * NX) nx = lds_frag(slot, li + xn, kn, lane);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = k; t < 6; ++t)
-            L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(di, dj[t - k], L[x][t], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        di = nx;
-    });
-}
-
-template <int NX>
-__device__ __forceinline__ void mul_w_a(i16v (&L)[NX][6], const std::uint8_t* slot, int li, int rj, int lane) {
-    i4 wj[6];
-    i4 wt = lds_frag(slot, li, 0, lane);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) wj[k] = lds_frag(slot, rj, k, lane);
-    const i4 vj = v_of_w0(wj[0]);
-    i4 vi{};
-    static_for<6 * NX>([&](auto ic) {
-        constexpr int i = decltype(ic)::value, x = i / 6, t = i % 6;
-        constexpr int xn = (i + 1) / 6, tn = (i + 1) % 6;
-        i4 nx = wt;
-        if constexpr (i + 1 < 6 * NX) nx = lds_frag(slot, li + xn, tn, lane);
-        if constexpr (t == 0) vi = v_of_w0(wt);
-        __builtin_amdgcn_sched_barrier(0);
-        L[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wt, vj, L[x][t], 0, 0, 0);
-        L[x][(t + 3) % 6] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vi, wj[(t + 3) % 6], L[x][(t + 3) % 6], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        wt = nx;
-    });
-}
-
 // One work item as a wavefront sees it (every field uniform): a block's K range, the tile's
 // row groups, and the wavefront's NX sub-tiles, left groups gI .. gI + NX - 1 (li in the
 // slot) against right group gJ (rj in the slot).
@@ -556,7 +513,7 @@ struct WaveItem {
 };
 
 // Every wavefront of the workgroup runs the same number of barriers whatever its NX.
-template <int NX, bool kAhead>
+template <int NX>
 __device__ __forceinline__ void run_item(const WaveItem& wi, const std::uint8_t* __restrict__ planes,
                                          std::int64_t KS32, int G32, int P, const double* __restrict__ vpair,
                                          double* __restrict__ f2, const FixupList& fl, std::uint8_t* lds_0,
@@ -602,14 +559,12 @@ __device__ __forceinline__ void run_item(const WaveItem& wi, const std::uint8_t*
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             stage_slot(src, slots[pf], offset(step + 1, 0), wave);
-            if constexpr (NX > 0 && kAhead) mul_q_a<NX>(L, slots[pd], wi.li, wi.rj, lane);
-            else if constexpr (NX > 0) mul_q_c<NX>(L, slots[pd], wi.li, wi.rj, lane);
+            if constexpr (NX > 0) mul_q<NX>(L, slots[pd], wi.li, wi.rj, lane);
             wait_vmcnt<kSetPlanes>();
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             stage_slot(src, slots[pd], offset(step + 1, 1), wave);
-            if constexpr (NX > 0 && kAhead) mul_w_a<NX>(L, slots[pw], wi.li, wi.rj, lane);
-            else if constexpr (NX > 0) mul_w_c<NX>(L, slots[pw], wi.li, wi.rj, lane);
+            if constexpr (NX > 0) mul_w<NX>(L, slots[pw], wi.li, wi.rj, lane);
         };
         if (seg0 > 0) __syncthreads();  // every reader of the previous segment's slots is done
         stage_slot(src, lds_0, offset(seg0, 0), wave);
@@ -667,7 +622,6 @@ __device__ __forceinline__ void run_item(const WaveItem& wi, const std::uint8_t*
     }
 }
 
-template <bool kAhead>
 __global__ __launch_bounds__(512) void f2_split_kernel(const std::uint8_t* __restrict__ planes, BlockTable bt,
                                                        const F2Item* __restrict__ items, ItemQueues queues,
                                                        unsigned* __restrict__ counters, int P, int G32,
@@ -715,9 +669,9 @@ __global__ __launch_bounds__(512) void f2_split_kernel(const std::uint8_t* __res
 #pragma unroll
         for (int x = 0; x < 2; ++x)
             n_act += wi.gI + x < G32 && wi.gJ < G32 && (!diag || wi.li + x <= wc);
-        if (n_act == 2) run_item<2, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
-        else if (n_act == 1) run_item<1, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
-        else run_item<0, kAhead>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
+        if (n_act == 2) run_item<2>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
+        else if (n_act == 1) run_item<1>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
+        else run_item<0>(wi, planes, KS32, G32, P, vpair, f2, fl, lds_0, lds_1, lds_2, wave, lane);
     }
     // The last item's look-ahead loads may still be landing in LDS: drain them before
     // the workgroup's LDS can be handed to another workgroup.
@@ -772,14 +726,11 @@ void launch_count_v8(const std::uint8_t* v8, BlockTable bt, const F2Item* items,
 
 void launch_f2_split(const std::uint8_t* planes, BlockTable bt, const F2Item* items, const ItemQueues& queues,
                      unsigned* counters, int P, int G32, std::int64_t KS32, const double* vpair, double* f2,
-                     const FixupList& fl, int n_workgroups, int ring, hipStream_t st) {
+                     const FixupList& fl, int n_workgroups, hipStream_t st) {
     if (queues.off[kXcds] <= 0) return;
     launch_zero_u32(counters, kXcds, st);
-    const dim3 grid(static_cast<unsigned>(n_workgroups));
-    if (ring == 1)
-        f2_split_kernel<true><<<grid, 512, 0, st>>>(planes, bt, items, queues, counters, P, G32, KS32, vpair, f2, fl);
-    else
-        f2_split_kernel<false><<<grid, 512, 0, st>>>(planes, bt, items, queues, counters, P, G32, KS32, vpair, f2, fl);
+    f2_split_kernel<<<static_cast<unsigned>(n_workgroups), 512, 0, st>>>(planes, bt, items, queues, counters, P, G32,
+                                                                         KS32, vpair, f2, fl);
     STP_LAUNCH_CHECK();
 }
 

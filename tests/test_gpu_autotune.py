@@ -19,8 +19,8 @@ from steppe_amd import _core, synth
 
 pytestmark = pytest.mark.gpu
 
-SPLIT_CANDIDATES = [f"sched={s},fp64_rows=64,fp64_prefetch=1,fp64_wg=2,count_wg={c},split_ring={g}"
-                    for g in (0, 1) for s in (0, 1) for c in (1, 2, 4)]
+SPLIT_CANDIDATES = [f"sched={s},fp64_rows=64,fp64_prefetch=1,fp64_wg=2,count_wg={c},split_ring=0"
+                    for s in (0, 1) for c in (1, 2, 4)]
 FP64_CANDIDATES = [f"sched={s},fp64_rows={r},fp64_prefetch={p},fp64_wg={w},count_wg=2,split_ring=0"
                    for s in (0, 1) for r in (64, 32) for p in (1, 0) for w in (1, 2, 3) if not (r == 64 and w == 3)]
 
@@ -101,4 +101,32 @@ def test_autotune_chooses_persists_and_is_used(engine, counts, tmp_path, monkeyp
         got = _f2(ctx2, counts, prec)
     finally:
         _core.lib().stp_close(ctx2.h)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+
+
+def test_table_of_an_earlier_version(engine, counts, tmp_path, monkeypatch):
+    # a saved choice that names the variant that is gone (split_ring=1) is read, its schedule
+    # and count grid used, and written back without it; one that names no known value is not
+    monkeypatch.delenv("STEPPE_F2_TUNE", raising=False)
+    panel, a2, n, ld = counts
+    prec = _core.STP_PREC_SPLIT_BF16
+    ref = _f2(engine, counts, prec)
+    P, nb = panel.n_pop, panel.n_block
+    f2, vp = torch.empty(P * P * nb, dtype=torch.float64, device="cuda"), torch.empty(P * P * nb, dtype=torch.float64,
+                                                                                      device="cuda")
+    old = "sched=1,fp64_rows=64,fp64_prefetch=1,fp64_wg=2,count_wg=4,split_ring="
+    cache = tmp_path / "f2_tune.tsv"
+    cache.write_text(f"some|other\t{old}1\nsome|thing\t{old}2\n")
+    monkeypatch.setenv("STEPPE_TUNE_CACHE", str(cache))
+    ctx = _core.Context(0)
+    try:
+        torch.cuda.synchronize()
+        _core.f2_autotune(ctx, a2.data_ptr(), n.data_ptr(), ld, P, panel.n_snp, panel.block_id, nb, prec,
+                          f2.data_ptr(), vp.data_ptr())
+        lines = dict(l.split("\t") for l in cache.read_text().splitlines())
+        assert lines["some|other"] == old + "0" and "some|thing" not in lines
+        monkeypatch.setenv("STEPPE_F2_TUNE", old + "1")
+        got = _f2(ctx, counts, prec)
+    finally:
+        _core.lib().stp_close(ctx.h)
     assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
