@@ -10,6 +10,7 @@
 // model's f4 basis reads each f2 series contiguously.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 #include <numeric>
 #include <vector>
 
@@ -241,8 +242,11 @@ void HipBackend::qpadm_small(QpFitArgs a, std::vector<QpLargeModel> models, cons
     constexpr std::size_t kBudget = std::size_t{1} << 29;        // doubles (4 GiB): setup results and weights
     constexpr std::size_t kMaxChunk = 16384;                     // models
     const int nbs = a.nbs;
+    // STEPPE_QPADM_REFITS=wave takes every refit with a wavefront a fit (tests).
+    const char* form = std::getenv("STEPPE_QPADM_REFITS");
+    const bool rows = !(form && std::strcmp(form, "wave") == 0);
     auto cls = [&](const QpLargeModel& md) {
-        return qpadm_rows_fit(md.nl, md.nr, md.rank, a.iters) ? qpadm_rows_class(md.nl, md.nr) : 0;
+        return rows && qpadm_rows_fit(md.nl, md.nr, md.rank, a.iters) ? qpadm_rows_class(md.nl, md.nr) : 0;
     };
     auto bucket = [&](const QpLargeModel& md) { return bucket_of(md.nl, md.nr, opt.rank); };
     // largest systems first: the launches that end in a few long fits come first

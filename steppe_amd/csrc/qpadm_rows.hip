@@ -17,9 +17,12 @@
 //   Seed    one-sided Jacobi on the columns: the rotations of the (p, q) loops that share
 //           p + q touch different columns and run at once, lane j with lane p + q - j.
 //
-// The estimator is als_fit's (qpadm.hip) operation for operation: every sum keeps its order,
-// products are rounded before they are added (no contraction), pivots and divisions are the
-// same, so the refits are als_fit's to the bit.  (A form with eliminations that need no
+// The estimator is als_fit's (qpadm.hip) operation for operation: the sums of a fit keep their
+// order, products are rounded before they are added (no contraction), pivots and divisions are
+// the same, so the refits are als_fit's to the bit, also for sources that can hardly be told
+// apart (compared over all shapes, up to 500 blocks).  Only the seed's stopping sum is added
+// per lane first: it falls by orders of magnitude from sweep to sweep, and where it met 1e-30
+// to within its rounding the seed could take a sweep more or less.  (A form with eliminations that need no
 // exchanges, contracted sums and Jacobi on the nl rows is twice as fast again, but its
 // standard errors differ by the rounding that near-degenerate models magnify: 1e-5.)
 //
