@@ -1,11 +1,14 @@
-"""The split form's digit bounds (steppe_amd/csrc/f2_split.hip, prep_split_kernel),
+"""The split form's digit bounds (steppe_amd/csrc/f2_split.hip, stage_entry and balanced48),
 restated in numpy from the kernel's own steps and checked against what the scheme needs:
 
-* q' = q - 1/2 as six balanced 8-bit digits: |d_0| <= 64, |d_k| <= 128 (exact in BF16);
-* w = -(q~^2 - h)/2 as four FP16 digits A, 32 b, 4 c, D on the levels with units 2^-14,
-  2^-30, 2^-38, 2^-46: each exactly representable in FP16 and |w - w~| <= 2^-47
-  (checked exactly with fractions on the worst cases);
-* per SNP, the growth of every FP32 level accumulator keeps 128 SNPs below 2^24.
+* q' = q - 1/2 and w = -(q~^2 - h)/2 as 48-bit integers in six balanced 8-bit digits:
+  |d_0| <= 64, every other digit in [-128, 127], |q~ - q'| <= 2^-48, |w~ - w| <= 2^-48;
+* the first w byte of an observed entry, W_0 + 96, has bit 6 set and bit 7 clear, so the flag
+  V = -128 v is its bit 6 moved up;
+* 16,384 SNPs keep every int32 level sum below 2^31, and the combined levels are exact in
+  64-bit integers and in a double;
+* the sum of the levels, with W_0's offset taken back from the pair count, is the estimator up
+  to the digits' truncation and the dropped products.
 
 Counts run over every population size of the panels (n = 1 .. 16383) with edge cases
 (q = 0, 1/2, 1 and q = 1/256-style values with short binary expansions).
@@ -14,78 +17,115 @@ from fractions import Fraction
 
 import numpy as np
 
+OFFSET = 96                # W_0' - W_0
+SEGMENT = 512 * 32         # SNPs summed in int32
 
-def _digits(a, n):
+
+def _balanced(x):
+    """Digits 0 (most significant) to 5 of round-to-even(x), by balanced48's bytes."""
+    bits = (x + 1.5 * 2.0 ** 52).view(np.uint64)
+    b = (bits + np.uint64(0x8080808080)) ^ np.uint64(0x8080808080)
+    return [((b >> np.uint64(8 * (5 - k))) & np.uint64(0xFF)).astype(np.uint8).view(np.int8).astype(np.int64)
+            for k in range(6)]
+
+
+def _entry(a, n):
+    """(d, W, q, w) of observed entries, as stage_entry forms them (W without its offset)."""
     q = a / (2.0 * n)
     h = q * (1.0 - q) / np.maximum(n - 1.0, 1.0)
-    x = (q - 0.5) * 128.0
-    d = []
-    for _ in range(6):
-        dk = np.rint(x)
-        d.append(dk)
-        x = (x - dk) * 256.0
-    qt = (d[0] + (d[1] + (d[2] + (d[3] + (d[4] + d[5] / 256) / 256) / 256) / 256) / 256) / 128
-    w = -0.5 * (qt * qt - h)
-    y = w * 16384.0
-    A = np.rint(y)
-    r1 = (y - A) * 2048.0
-    b = np.rint(r1)
-    r2 = (r1 - b) * 2048.0
-    c = np.rint(r2)
-    D = np.rint((r2 - c) * 1024.0)
-    return d, w, A, 32.0 * b, 4.0 * c, D
+    assert (h >= 0).all()
+    x = (q - 0.5) * 2.0 ** 47
+    qt = ((x + 1.5 * 2.0 ** 52) - 1.5 * 2.0 ** 52) * 2.0 ** -47
+    y = qt * qt - h
+    return _balanced(x), _balanced(y * 2.0 ** 46), q, -0.5 * y
 
 
-def _counts():
+def _value(d):
+    return sum(dk << (8 * (5 - k)) for k, dk in enumerate(d))
+
+
+def _counts(size=1_000_000):
     rng = np.random.default_rng(7)
-    n = rng.integers(1, 16384, 2_000_000).astype(np.float64)
+    n = rng.integers(1, 16384, size).astype(np.float64)
     a = np.minimum(np.floor(rng.random(n.size) * (2 * n + 1)), 2 * n)
     edge_n = np.array([1, 1, 1, 2, 2, 128, 128, 16383, 16383, 16383, 256, 512], np.float64)
     edge_a = np.array([0, 1, 2, 1, 3, 1, 255, 0, 16383, 32766, 1, 3], np.float64)
     return np.concatenate([edge_a, a]), np.concatenate([edge_n, n])
 
 
-def test_q_digits_fit_bf16():
-    a, n = _counts()
-    d, *_ = _digits(a, n)
+def test_q_digits():
+    d, _, q, _ = _entry(*_counts())
     assert np.abs(d[0]).max() <= 64
-    for dk in d[1:]:
-        assert np.abs(dk).max() <= 128
-    # integers with at most 8 significant bits are exact in BF16 (and d5 / 256 too)
-    for dk in d:
-        f = dk.astype(np.float32).view(np.uint32)
-        assert np.all(f & 0xFFFF == 0)
-
-
-def test_w_digits_fit_fp16_and_reconstruct_w():
-    a, n = _counts()
-    _, w, A, B, C, D = _digits(a, n)
-    assert np.abs(A).max() <= 2048 and np.abs(B).max() <= 32 * 1024
-    assert np.abs(C).max() <= 4 * 1024 and np.abs(D).max() <= 512
-    for v in (A, B, C, D):
-        assert np.array_equal(v.astype(np.float16).astype(np.float64), v)
-    wt = A * 2.0 ** -14 + B * 2.0 ** -30 + C * 2.0 ** -38 + D * 2.0 ** -46
-    err = np.abs(w - wt)
-    assert err.max() <= 2.0 ** -47 * (1 + 1e-9)
+    err = np.abs(_value(d) * 2.0 ** -47 - (q - 0.5))
+    assert err.max() <= 2.0 ** -48
+    # (against q itself, the subtraction's rounding of at most 2^-55 comes on top)
     for i in np.argsort(err)[-20:]:
-        exact = (Fraction(int(A[i]), 2 ** 14) + Fraction(int(B[i]), 2 ** 30) + Fraction(int(C[i]), 2 ** 38)
-                 + Fraction(int(D[i]), 2 ** 46))
-        assert abs(Fraction(float(w[i])) - exact) <= Fraction(1, 2 ** 47)
+        exact = Fraction(float(q[i])) - Fraction(1, 2)
+        assert abs(Fraction(int(_value(d)[i]), 2 ** 47) - exact) <= Fraction(1, 2 ** 48) + Fraction(1, 2 ** 55)
 
 
-def test_level_accumulators_stay_exact_over_128_snps():
-    a, n = _counts()
-    d, _, A, B, C, D = _digits(a, n)
-    m = [np.abs(x).max() for x in d]
-    # worst case per SNP: the largest digits on both sides of every product of a level
-    levels = [
-        m[0] * m[0] + 2 * np.abs(A).max(),
-        2 * m[0] * m[1],
-        2 * m[0] * m[2] + m[1] * m[1] + 2 * np.abs(B).max(),
-        2 * m[0] * m[3] + 2 * m[1] * m[2] + 2 * np.abs(C).max(),
-        2 * m[0] * m[4] + 2 * m[1] * m[3] + m[2] * m[2]
-        + (2 * m[0] * m[5] + 2 * m[1] * m[4] + 2 * m[2] * m[3]) / 256 + 2 * np.abs(D).max(),
-    ]
-    for t, g in enumerate(levels):
-        # 128 SNPs plus the carry a level receives from the one below it (< 2^16)
-        assert 128 * g + 2 ** 16 < 2 ** 24, (t, g)
+def test_w_digits_and_the_flag():
+    _, W, _, w = _entry(*_counts())
+    byte = W[0] + OFFSET
+    assert byte.min() >= 79 and byte.max() <= 113
+    assert ((byte & 0x40) == 0x40).all() and ((byte & 0x80) == 0).all()
+    assert (((byte << 1) & 0x80).astype(np.uint8).view(np.int8) == -128).all() and (0 << 1) & 0x80 == 0
+    # w~ = -128 sum_k W_k 2^(-14 - 8 k)
+    exact = [Fraction(-int(v), 2 ** 47) for v in _value(W)[:20]]
+    got = -_value(W) * 2.0 ** -47
+    assert all(Fraction(float(g)) == e for g, e in zip(got, exact))
+    err = np.abs(got - w)
+    assert err.max() <= 2.0 ** -48
+    for i in np.argsort(err)[-20:]:
+        assert abs(Fraction(-int(_value(W)[i]), 2 ** 47) - Fraction(float(w[i]))) <= Fraction(1, 2 ** 48)
+
+
+def test_level_sums_fit_int32():
+    d, W, _, _ = _entry(*_counts())
+    m = [int(np.abs(x).max()) for x in d]
+    W[0] = W[0] + OFFSET
+    growth = [sum(m[k] * m[t - k] for k in range(t + 1)) + 2 * 128 * int(np.abs(W[t]).max()) for t in range(6)]
+    assert max(growth) == growth[5] <= 114_688
+    assert all(SEGMENT * g < 2 ** 31 for g in growth)
+    # the epilogue's upper and lower halves, exact in a double
+    level = [SEGMENT * g for g in growth]
+    level[0] += 2 * 128 * OFFSET * SEGMENT
+    assert (level[0] << 16) + (level[1] << 8) + level[2] < 2 ** 53
+    assert (level[3] << 16) + (level[4] << 8) + level[5] < 2 ** 53
+
+
+def test_levels_recombine_to_the_estimator():
+    # a block of 3 segments, two populations with missing entries: levels summed in integers,
+    # W_0's offset taken back in shares of the pair count
+    rng = np.random.default_rng(3)
+    M = 2 * SEGMENT + 77
+    ent, v = [], []
+    for _ in range(2):
+        n = rng.integers(1, 60, M).astype(np.float64)
+        ent.append(_entry(np.floor(rng.random(M) * (2 * n + 1)), n))
+        v.append((rng.random(M) < np.where(np.arange(M) < SEGMENT, 0.3, 0.95)).astype(np.int64))
+    (di, Wi, qi, wi), (dj, Wj, qj, wj) = ent
+    vi, vj = v
+    steps = -(-M // 64) * 2                       # blocks are padded to 64 SNPs
+    pairs = int((vi * vj).sum())
+    num = Fraction(0)
+    for s0 in range(0, steps, 512):
+        s1 = min(s0 + 512, steps)
+        at = slice(32 * s0, min(32 * s1, M))
+        L = []
+        for t in range(6):
+            x = sum((di[k] * dj[t - k] * vi * vj)[at].sum() for k in range(t + 1))
+            wt, wu = (Wi[t] + (OFFSET if t == 0 else 0)) * vi, (Wj[t] + (OFFSET if t == 0 else 0)) * vj
+            L.append(int(x + (-128 * vj * wt)[at].sum() + (-128 * vi * wu)[at].sum()))
+            assert abs(L[-1]) < 2 ** 31
+        L[0] += 2 * 128 * OFFSET * (pairs * s1 // steps - pairs * s0 // steps)
+        hi, lo = (L[0] << 16) + (L[1] << 8) + L[2], (L[3] << 16) + (L[4] << 8) + L[5]
+        num += -2 * (Fraction(hi, 2 ** 30) + Fraction(lo, 2 ** 54))
+    want = Fraction(0)
+    both = np.flatnonzero(vi * vj)
+    for s in both:
+        x, y = Fraction(float(qi[s])) - Fraction(1, 2), Fraction(float(qj[s])) - Fraction(1, 2)
+        want += -2 * (x * y + Fraction(float(wi[s])) + Fraction(float(wj[s])))
+    # per SNP: two digit truncations of at most 2^-48 on each operand and products k + l >= 6
+    assert abs(num - want) <= len(both) * Fraction(1, 2 ** 43)
+    print(f"  {len(both)} pairs: off by {float(abs(num - want)) / len(both):.1e} a pair")
