@@ -40,7 +40,7 @@ extern "C" {
 
 /* f2 arithmetic forms (reference: steppe::Precision, include/steppe/config.hpp:74-110). */
 #define STP_PREC_FP64 0        /* FP64 MFMA contraction                                 */
-#define STP_PREC_SPLIT_BF16 1  /* fixed-point BF16 slices on BF16 MFMA, FP64 recombination */
+#define STP_PREC_SPLIT_BF16 1  /* 48-bit fixed point in 8-bit digits on int8 MFMA, FP64 recombination */
 
 typedef struct stp_context stp_context;
 typedef struct stp_f2_handle stp_f2_handle;

@@ -31,8 +31,8 @@ constexpr int kTileRows = 64;  // rows per wavefront output tile (4 row groups)
 // Split form: 12 one-byte digit planes per (population, SNP) (f2_split.hip).
 constexpr int kSplitPlanes = 12;
 // Bytes per (population, SNP) that the automatic output tier counts for the split form's
-// working set: more than the planes take, kept so that a panel's tier does not depend on
-// how the digits are laid out.
+// planes.  They take 12; 22 is what it has always counted (an earlier layout's), kept as an
+// upper bound so that no panel changes its tier, and with it what its handle accepts.
 constexpr int kSplitTierBytes = 22;
 
 struct BlockTable {

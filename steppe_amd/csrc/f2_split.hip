@@ -41,10 +41,12 @@
 // digits, then the w digits) whose 48 KB of planes arrive in a ring of three LDS slots
 // by direct global->LDS loads, issued two phases ahead.
 //
-// Bound and measured (1000 populations x 597,573 SNPs, one pass): the contraction issues
-// 33 x 2 ops per pair-SNP of its 128-row tiles, 2.3e13 in 9.2 ms = 2.5 POP/s, the rate an
-// 8192^3 int8 library product reaches on this card (2.49); on the BF16 / FP16 digits it
-// took 18.3 ms.  Prep writes 12 instead of 23 bytes per entry: 2.0 instead of 4.5 ms.
+// Bound and measured: the contraction issues 33 x 2 ops per output and SNP of its sub-tiles
+// (blocks padded to 64 SNPs; of a diagonal tile ten of sixteen sub-tiles), 1.10 times those of
+// the population pairs.  1000 populations x 1.2M SNPs: 4.36e13 ops in 18.6 ms = 2.34 POP/s
+// with the matrix pipes busy 64% of the cycles, 94% of the rate that a plain 8192^3 int8
+// library product reaches on this card (2.49); 1000 x 597,573: 9.2 ms, on the BF16 / FP16
+// digits 18.3.  Prep writes 12 instead of 23 bytes per entry: 2.0 instead of 4.5 ms.
 
 #include <utility>
 

@@ -379,16 +379,16 @@ __device__ __noinline__ bool als_fit(const double* Q, int ldq_arg, FitShape s_ar
 }
 
 // ---------------------------------------------------------------------------------
-// the batched kernel
+// the batched kernels
 // ---------------------------------------------------------------------------------
-// Wavefronts per SIMD each system-size bucket is compiled for.  The fits are bound by
-// the latency of their lane reads, LDS accesses and short dependent FP64 chains, not by
-// register traffic: capping the registers (what does not fit spills to scratch) for
-// more resident wavefronts is faster.  On the 10,000-model C4 fleet: no cap 1,923
-// fits/s; 4 for T = 16, 3 for T = 32: 2,244; 4 for T <= 32 and 3 for T = 48: 2,654;
-// 4 for T = 48: 2,604; 5 for T = 32: 2,494; with the fit's sizes in scalar registers,
-// 4 / 4 / 3: 2,885 and 5 / 4 / 3: 2,925 (two runs each; eight wavefronts per workgroup
-// instead of four: 2,690).
+// Wavefronts per SIMD each system-size bucket is compiled for.  The fits are bound by the
+// latency of their lane reads, LDS accesses and short dependent FP64 chains, not by register
+// traffic: capping the registers (what does not fit spills to scratch) for more resident
+// wavefronts is faster where many fits run at once.  The fit tables of 1330 models of 2-3
+// sources and 8 right populations, beside their refits: whole call 31.5 ms with 5 for T = 16,
+// 33.9 with 4, 33.7 without a cap.  For T = 32 and 48 the tables of 1000 mixed models hide
+// behind the refits (7.8 and 12.9 ms of 157; without caps 7.3 and 12.5, the call 159): 4 and 3
+// stand for calls whose refits run here too.
 template <int T>
 constexpr int qpadm_waves_per_simd() {
     return T == 16 ? 5 : (T == 32 ? 4 : (T == 48 ? 3 : 1));

@@ -122,9 +122,9 @@ void launch_qpadm_setup(const QpFitArgs& g, int n_models, int m_max, hipStream_t
 // The fits of one system-size bucket T by wavefronts with a matrix row per lane: each
 // model's fit table, or (refits) its leave-one-block-out refits.
 void launch_qpadm_fits(int T, const QpFitArgs& g, bool refits, int n_models, int m_max, int nr_max, hipStream_t st);
-// Leave-one-block-out refits with sixteen lanes a fit: whether a model's take that form, the
-// kernel instance, and the launch over models of one instance (g.models, g.tables and g.wm
-// at the chunk's first model plus slot0).
+// Leave-one-block-out refits with eight or sixteen lanes a fit: whether a model's take that
+// form, the kernel instance, and the launch over models of one instance (g.models and g.tables
+// at its first model, g.wm at the chunk's first).
 bool qpadm_rows_fit(int nl, int nr, int rank, int iters);
 int qpadm_rows_class(int nl, int nr);
 void launch_qpadm_rows(const QpFitArgs& g, int cls, int n_models, int m_max, hipStream_t st);

@@ -5,7 +5,7 @@
 // src/device/cuda/cuda_backend_qpadm_fit.cu:623-960 and run_qpadm_search,
 // src/core/qpadm/model_search.cpp:30-218): survivor blocks are found once for the
 // tensor, models are validated and grouped by the size of their largest normal
-// matrix, and each group runs as one persistent launch; results come back in input
+// matrix, and each stage of the fit is one launch per group; results come back in input
 // order.  The f2 slab is first transposed to pair-major, survivor-only order so a
 // model's f4 basis reads each f2 series contiguously.
 #include <algorithm>
@@ -162,9 +162,7 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
     const std::size_t o_surv = put(surv.data(), surv.size());
     const std::size_t o_bsz = put(bsz.data(), bsz.size());
     const std::size_t o_tgt = put(target, n_models);
-    const std::size_t o_loff = put(left_off, n_models + 1);
     const std::size_t o_left = put(left, total_left);
-    const std::size_t o_roff = put(right_off, n_models + 1);
     const std::size_t o_right = put(right, total_right);
     qp_i32_.ensure(arena.size());
     STP_HIP(hipMemcpyAsync(qp_i32_.get(), arena.data(), arena.size() * sizeof(std::int32_t), hipMemcpyHostToDevice,
@@ -174,7 +172,7 @@ void HipBackend::qpadm_batch(const F2Blocks& h, int n_models, const std::int32_t
     qpT_.ensure(static_cast<std::size_t>(slab) * nbs);
     launch_transpose_survivors(h.f2.get(), slab, qp_i32_.get() + o_surv, nbs, qpT_.get(), stream_);
 
-    // ---- launches per bucket ----
+    // ---- the fits ----
     qp_out_.ensure(static_cast<std::size_t>(n_models));
     STP_HIP(hipMemsetAsync(qp_out_.get(), 0, static_cast<std::size_t>(n_models) * sizeof(stp_qpadm_result), stream_));
     mark_begin(kQpadm);

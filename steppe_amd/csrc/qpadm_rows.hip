@@ -31,7 +31,8 @@
 // models of 2-5 sources and 6-12 right populations 1,061 ms as a workgroup per model and a
 // wavefront per fit, 165 ms so (the whole call; 204 ms with 16 lanes for every fit, which
 // leaves half of them idle up to 8 columns); a rotation of 1330 models of 2-3 sources against
-// 8 right populations 242 -> 31 ms (51); one model of 2 sources 43.5 -> 0.58 ms.  Columns
+// 8 right populations 242 -> 31.5 ms (51; without the garbage collections of its 1330 result
+// dicts, which add up to 45 ms to a call now and then); one model of 2 sources 43.5 -> 0.58 ms.  Columns
 // padded to 6, 8, 10, 12 with straight-line sums instead of a test per column: the same time
 // at 3 sources, 2.3 times slower at 5 (spills).
 

@@ -126,7 +126,7 @@ void HostArray::alloc(std::size_t n) {
 std::size_t f2_working_set_bytes(const F2Plan& plan, int precision) {
     const std::size_t K = static_cast<std::size_t>(plan.K_total);
     const std::size_t rows16 = static_cast<std::size_t>(plan.G) * kRowGroup;
-    const std::size_t v8 = rows16 * K;   // int8 V plane
+    const std::size_t v8 = rows16 * K;   // the FP64 form's int8 V plane (counted for both)
     const std::size_t planes = precision == STP_PREC_FP64 ? 3 * sizeof(double) * rows16 * K
                                                           : kSplitTierBytes * static_cast<std::size_t>(plan.G32) * 32 * K;
     const std::size_t upper = static_cast<std::size_t>(plan.P) * (plan.P + 1) / 2 * plan.n_block;
@@ -153,8 +153,8 @@ F2Blocks* HipBackend::f2_counts_tiered(const std::uint16_t* a2, const std::uint1
     const F2Plan full = make_f2_plan(P, M, block_id, n_block);   // validates the partition
     int tier = tr.tier;
     if (tier < 0) {
-        // resident only when the result and the contraction's working set (planes, int8 V
-        // plane, fix-up list) fit together, as the reference's select_output_tier adds
+        // resident only when the result and an upper bound of the contraction's working set
+        // (planes, fix-up list) fit together, as the reference's select_output_tier adds
         // its resident working set (src/device/tier_select.hpp:62-72)
         tier = choose_f2_tier(result_bytes, f2_working_set_bytes(full, precision), free_vram, free_host_bytes());
     }

@@ -1,4 +1,4 @@
-"""GPU parity of the split-BF16 f2 form (fixed-point BF16 slices on BF16 MFMA).
+"""GPU parity of the split f2 form (48-bit fixed point in 8-bit digits on int8 MFMA).
 
 Bar: vpair bit-exact; f2 within 1e-9 relative of the FP64 oracle with an absolute
 floor of 1e-6 f2 units on |r| (|c - r| <= 1e-9 * max(|r|, 1e-6)) — the tolerance
@@ -60,8 +60,7 @@ def test_split_population_counts_edge_cases(engine, cref, P):
 
 def test_split_long_blocks_and_extreme_frequencies(engine, cref):
     # 8000-SNP blocks (the largest the workloads allow) with frequencies pinned at
-    # 0 and 1 in half the populations: the carry chain and the level bounds at
-    # their worst case.
+    # 0 and 1 in half the populations: the digits and the level sums near their bounds.
     rng = np.random.default_rng(5)
     P, M = 40, 16000
     q = rng.random((P, M))
